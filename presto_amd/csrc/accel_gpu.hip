@@ -9,8 +9,8 @@
  *       wavefront per window by ballot counts for windows of <= 1024
  *       bins, a workgroup radix select in LDS above) and the block-median
  *       normalisation of src/accel_utils.c:1087-1099.
- *   k_corr4096 : fused overlap-save correlation -- spread spectrum
- *       segment -> Stockham radix-16 FFT in LDS -> multiply by each
+ *   k_corr : fused overlap-save correlation -- spectrum
+ *       segment -> Stockham FFT in LDS -> multiply by each
  *       template -> inverse FFT -> |.|^2 -> raw plane row
  *       (the template loop of src/accel_utils.c:1141-1190).
  *   k_harmsum : harmonic summing with the reference's index rules and
@@ -49,6 +49,8 @@ static int fail(const char *msg)
 }
 
 #include "dev_fresnel.h"
+
+#define CORR_N 4096   /* half-bins per correlation segment */
 
 /* One tap of the z-response kernel with roffset = 0 and numbetween = 2
  * (src/responses.c:159-225 for |z| < 1e-4, :228-316 otherwise). */
@@ -139,31 +141,48 @@ __global__ __launch_bounds__(256) void k_resp_w(const int *zs, const int *ws, co
     }
 }
 
-/* T[t][f] = conj(sum_m resp[nk/2+m] e^{-2 pi i f m / L}) / L in FP64 */
-__global__ void k_template_dft(const double2 *resp, const int *nks, int nkmax, int L,
-                               float2 *T)
+/* Correlation templates for segments of L = 4096 half-bins whose odd
+ * half-bins are zero.  With T[f] = conj(sum_m resp[nk/2+m]
+ * e^{-2 pi i f m / L}) / L, the even and the odd half-bins of the
+ * correlation are inverse transforms of half the length, of
+ *   Te[f] = T[f] + T[f + L/2]                       (the even taps)
+ *   To[f] = (T[f] - T[f + L/2]) e^{2 pi i f / L}    (the odd taps)
+ * times the data's transform.  Both in FP64, rounded to FP32, stored in
+ * the order in which k_corr reads them: a thread's pairs f = j + 128 p,
+ * f + 1024 side by side. */
+__global__ void k_template_dft(const double2 *resp, const int *nks, int nkmax, float2 *T)
 {
+    const int L = CORR_N;
     const int t = blockIdx.y;
     const int f = blockIdx.x * blockDim.x + threadIdx.x;
-    if (f >= L)
+    if (f >= L / 2)
         return;
-    const int nk = nks[t], half = nk / 2;
+    const int nk = nks[t], half = nk / 2;   /* half is even */
     const double2 *rp = resp + (size_t) t * nkmax;
-    double ws, wc, s0, c0;
-    sincospi(-2.0 * (double) f / (double) L, &ws, &wc);
-    long long e0 = ((long long) f * half) % L;              /* m = -half */
+    double ws, wc, s0, c0, s1, c1;
+    sincospi(-4.0 * (double) f / (double) L, &ws, &wc);    /* two taps on */
+    sincospi(2.0 * (double) f / (double) L, &s1, &c1);
+    const int e0 = (int) (((long long) f * half) % L);     /* m = -half */
     sincospi(2.0 * (double) e0 / (double) L, &s0, &c0);
-    double cr = c0, ci = s0, ar = 0.0, ai = 0.0;
-    for (int m = 0; m < nk; m++) {
-        double2 v = rp[m];
-        ar += v.x * cr - v.y * ci;
-        ai += v.x * ci + v.y * cr;
-        double nr = cr * wc - ci * ws;
+    double cr = c0, ci = s0, er = 0.0, ei = 0.0, odr = 0.0, odi = 0.0;
+    for (int m = 0; m < nk; m += 2) {
+        const double2 v = rp[m], u = rp[m + 1];
+        er += v.x * cr - v.y * ci;
+        ei += v.x * ci + v.y * cr;
+        odr += u.x * cr - u.y * ci;   /* without the odd tap's own e^{-2 pi i f / L} */
+        odi += u.x * ci + u.y * cr;
+        const double nr = cr * wc - ci * ws;
         ci = cr * ws + ci * wc;
         cr = nr;
     }
-    const double inv = 1.0 / (double) L;
-    T[(size_t) t * L + f] = make_float2((float) (ar * inv), (float) (-ai * inv));
+    /* conj(sum_odd e^{-2 pi i f / L}) e^{2 pi i f / L} = conj(sum_odd) e^{4 pi i f / L} */
+    const double inv = 2.0 / (double) L;
+    const int j = f & 127, r = f >> 7;
+    float2 *o = T + (size_t) t * L + (r & 7) * 256 + 2 * j + (r >> 3);
+    o[0] = make_float2((float) (er * inv), (float) (-ei * inv));
+    const double tr = c1 * c1 - s1 * s1, ti = 2.0 * c1 * s1;
+    o[L / 2] = make_float2((float) ((odr * tr + odi * ti) * inv),
+                           (float) ((odr * ti - odi * tr) * inv));
 }
 
 /* ------------------------------------------------------------------ */
@@ -518,121 +537,191 @@ __global__ void k_inmem_nsq_table(const float *nsq, int npre, int nblocks, long 
 }
 
 /* ------------------------------------------------------------------ */
-/* Stockham radix-16 FFT of length 4096 over 256 threads               */
+/* Overlap-save correlation                                             */
 /* ------------------------------------------------------------------ */
-__device__ __forceinline__ float2 cadd(float2 a, float2 b) { return make_float2(a.x + b.x, a.y + b.y); }
-__device__ __forceinline__ float2 csub(float2 a, float2 b) { return make_float2(a.x - b.x, a.y - b.y); }
-__device__ __forceinline__ float2 cmul(float2 a, float2 w)
+
+/* Butterflies (a, b) -> (a + t b, a - t b), the twiddle product fused into
+ * the sum: four multiply-adds give a + t b, two more 2 a - (a + t b). */
+__device__ __forceinline__ void bfly(float2 &a, float2 &b, float2 t)
 {
-    return make_float2(a.x * w.x - a.y * w.y, a.x * w.y + a.y * w.x);
+    const float x = __builtin_fmaf(-b.y, t.y, __builtin_fmaf(b.x, t.x, a.x));
+    const float y = __builtin_fmaf(b.x, t.y, __builtin_fmaf(b.y, t.x, a.y));
+    b = make_float2(__builtin_fmaf(2.0f, a.x, -x), __builtin_fmaf(2.0f, a.y, -y));
+    a = make_float2(x, y);
 }
 
-/* 4-point DFT with W4 = S*i */
-template <int S>
-__device__ __forceinline__ void dft4(float2 &a0, float2 &a1, float2 &a2, float2 &a3)
+/* the twiddle i t */
+__device__ __forceinline__ void bfly_i(float2 &a, float2 &b, float2 t)
 {
-    float2 s02 = cadd(a0, a2), d02 = csub(a0, a2);
-    float2 s13 = cadd(a1, a3), d13 = csub(a1, a3);
-    float2 e = make_float2(-S * d13.y, S * d13.x);
-    a0 = cadd(s02, s13);
-    a2 = csub(s02, s13);
-    a1 = cadd(d02, e);
-    a3 = csub(d02, e);
+    const float x = __builtin_fmaf(-b.x, t.y, __builtin_fmaf(-b.y, t.x, a.x));
+    const float y = __builtin_fmaf(-b.y, t.y, __builtin_fmaf(b.x, t.x, a.y));
+    b = make_float2(__builtin_fmaf(2.0f, a.x, -x), __builtin_fmaf(2.0f, a.y, -y));
+    a = make_float2(x, y);
 }
 
-/* 16-point DFT as 4x4: X[c+4d] ends in slot 4c+d */
-template <int S>
-__device__ __forceinline__ void dft16(float2 *v)
+/* the twiddles 1 and i */
+__device__ __forceinline__ void bfly1(float2 &a, float2 &b)
 {
-    const float C1 = 0.92387953251128675613f, S1 = 0.38268343236508977173f;
-    const float R2 = 0.70710678118654752440f;
+    const float2 d = make_float2(a.x - b.x, a.y - b.y);
+    a = make_float2(a.x + b.x, a.y + b.y);
+    b = d;
+}
+__device__ __forceinline__ void bfly1_i(float2 &a, float2 &b)
+{
+    const float2 d = make_float2(a.x + b.y, a.y - b.x);
+    a = make_float2(a.x - b.y, a.y + b.x);
+    b = d;
+}
+
+/* Inverse-sign DFTs of v[r] w^r, radix 2, decimation in time, in place:
+ * X[k] ends in slot bitrev(k).  The twiddles of every stage come from a
+ * few powers of w (the factors i are free). */
+#define REV8(k) ((((k) & 1) << 2) | ((k) & 2) | (((k) >> 2) & 1))
+#define REV16(k) ((((k) & 1) << 3) | (((k) & 2) << 1) | (((k) >> 1) & 2) | (((k) >> 3) & 1))
+
+/* w = 1, after the first stage (the pairs r, r + 8) */
+__device__ __forceinline__ void dft16_rest(float2 *v)
+{
+    const float2 w1 = make_float2(0.92387953251128675613f, 0.38268343236508977173f);
+    const float2 w2 = make_float2(0.70710678118654752440f, 0.70710678118654752440f);
+    const float2 w3 = make_float2(0.38268343236508977173f, 0.92387953251128675613f);
 #pragma unroll
-    for (int b = 0; b < 4; b++)
-        dft4<S>(v[b], v[4 + b], v[8 + b], v[12 + b]);
-    /* slot 4c+b *= W16^(b c) */
-    v[5] = cmul(v[5], make_float2(C1, S * S1));                              /* W^1 */
-    v[9] = make_float2(R2 * (v[9].x - S * v[9].y), R2 * (S * v[9].x + v[9].y));   /* W^2 (b1,c2) */
-    v[13] = cmul(v[13], make_float2(S1, S * C1));                            /* W^3 */
-    v[6] = make_float2(R2 * (v[6].x - S * v[6].y), R2 * (S * v[6].x + v[6].y));   /* W^2 (b2,c1) */
-    v[10] = make_float2(-S * v[10].y, S * v[10].x);                          /* W^4 */
-    v[14] = make_float2(R2 * (-v[14].x - S * v[14].y), R2 * (S * v[14].x - v[14].y)); /* W^6 */
-    v[7] = cmul(v[7], make_float2(S1, S * C1));                              /* W^3 */
-    v[11] = make_float2(R2 * (-v[11].x - S * v[11].y), R2 * (S * v[11].x - v[11].y)); /* W^6 */
-    v[15] = cmul(v[15], make_float2(-C1, -S * S1));                          /* W^9 */
+    for (int r = 0; r < 4; r++) {
+        bfly1(v[r], v[r + 4]);
+        bfly1_i(v[r + 8], v[r + 12]);
+    }
 #pragma unroll
-    for (int c = 0; c < 4; c++)
-        dft4<S>(v[4 * c], v[4 * c + 1], v[4 * c + 2], v[4 * c + 3]);
+    for (int r = 0; r < 2; r++) {
+        bfly1(v[r], v[r + 2]);
+        bfly(v[r + 8], v[r + 10], w2);
+        bfly1_i(v[r + 4], v[r + 6]);
+        bfly_i(v[r + 12], v[r + 14], w2);
+    }
+    bfly1(v[0], v[1]);
+    bfly(v[8], v[9], w1);
+    bfly(v[4], v[5], w2);
+    bfly(v[12], v[13], w3);
+    bfly1_i(v[2], v[3]);
+    bfly_i(v[10], v[11], w1);
+    bfly_i(v[6], v[7], w2);
+    bfly_i(v[14], v[15], w3);
 }
 
-#define OUTSLOT(k) (4 * ((k) & 3) + ((k) >> 2))
+/* t: w^8, w^4, w^2, w^2 W8, w, w W16, w W8, w W16^3 */
+__device__ __forceinline__ void dft16_tw(float2 *v, const float2 *t)
+{
+#pragma unroll
+    for (int r = 0; r < 8; r++)
+        bfly(v[r], v[r + 8], t[0]);
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+        bfly(v[r], v[r + 4], t[1]);
+        bfly_i(v[r + 8], v[r + 12], t[1]);
+    }
+#pragma unroll
+    for (int r = 0; r < 2; r++) {
+        bfly(v[r], v[r + 2], t[2]);
+        bfly(v[r + 8], v[r + 10], t[3]);
+        bfly_i(v[r + 4], v[r + 6], t[2]);
+        bfly_i(v[r + 12], v[r + 14], t[3]);
+    }
+    bfly(v[0], v[1], t[4]);
+    bfly(v[8], v[9], t[5]);
+    bfly(v[4], v[5], t[6]);
+    bfly(v[12], v[13], t[7]);
+    bfly_i(v[2], v[3], t[4]);
+    bfly_i(v[10], v[11], t[5]);
+    bfly_i(v[6], v[7], t[6]);
+    bfly_i(v[14], v[15], t[7]);
+}
+
+/* t: w^4, w^2, w, w W8 */
+__device__ __forceinline__ void dft8_tw(float2 *v, const float2 *t)
+{
+#pragma unroll
+    for (int r = 0; r < 4; r++)
+        bfly(v[r], v[r + 4], t[0]);
+#pragma unroll
+    for (int r = 0; r < 2; r++) {
+        bfly(v[r], v[r + 2], t[1]);
+        bfly_i(v[r + 4], v[r + 6], t[1]);
+    }
+    bfly(v[0], v[1], t[2]);
+    bfly(v[4], v[5], t[3]);
+    bfly_i(v[2], v[3], t[2]);
+    bfly_i(v[6], v[7], t[3]);
+}
+
+/* e^{2 pi i a / n}, FP64 rounded to FP32 */
+__device__ static float2 unit_root(int a, int n)
+{
+    double s, c;
+    sincospi(2.0 * (double) a / (double) n, &s, &c);
+    return make_float2((float) c, (float) s);
+}
+
+/* LDS slot of point i: one slot of padding every 16.  LPR(i, r): of point
+ * i + r, r a multiple of 16 (an immediate offset from i's slot) */
 #define LP(i) ((i) + ((i) >> 4))
-#define FFT_LDS (4096 + 256)
+#define LPR(i, r) (LP(i) + (r) + (r) / 16)
+#define FFT_HALF (CORR_N / 2)
+#define FFT_LDS (FFT_HALF + FFT_HALF / 16)
 
-/* Input v[r] = x[j + 256 r]; output v[r] = X[j + 256 r].  tw1l is the
- * LDS table W_256^{r m} at [16 r + m] (m = j % 16, the first inter-pass
- * twiddles); tw2 holds this thread's second inter-pass twiddles
- * W_4096^{r j}.  Twiddles are the inverse-sign (S = +1) values. */
-template <int S>
-__device__ __forceinline__ void fft4096(float2 *v, float2 *lds, const float2 *tw1l,
-                                        const float2 *tw2)
+/* The two exchanges of an inverse FFT of 2048 points by 128 threads (16
+ * points each, radix 16, 16, 8): v holds the first radix-16 DFT's output
+ * in REV16 order; on return buf holds the input of the radix-8 pass.
+ * Called by the whole workgroup, each half on its own buf. */
+__device__ __forceinline__ void fft2048_mid(float2 *v, float2 *buf, int j, const float4 *tw2)
 {
-    const int j = threadIdx.x;
-    dft16<S>(v);
 #pragma unroll
     for (int r = 0; r < 16; r++)
-        lds[LP(16 * j + r)] = v[OUTSLOT(r)];
+        buf[LP(16 * j) + r] = v[REV16(r)];
     __syncthreads();
 #pragma unroll
     for (int r = 0; r < 16; r++)
-        v[r] = lds[LP(j + 256 * r)];
-    __syncthreads();
+        v[r] = buf[LPR(j, 128 * r)];
+    float2 tw[8];
 #pragma unroll
-    for (int r = 1; r < 16; r++) {
-        float2 w = tw1l[16 * r + (j & 15)];
-        v[r] = cmul(v[r], make_float2(w.x, S * w.y));
+    for (int r = 0; r < 4; r++) {
+        const float4 w = tw2[r];
+        tw[2 * r] = make_float2(w.x, w.y);
+        tw[2 * r + 1] = make_float2(w.z, w.w);
     }
-    dft16<S>(v);
-    const int base1 = (j >> 4) * 256 + (j & 15);
-#pragma unroll
-    for (int r = 0; r < 16; r++)
-        lds[LP(base1 + 16 * r)] = v[OUTSLOT(r)];
     __syncthreads();
+    dft16_tw(v, tw);
+    const int base = (j >> 4) * 256 + (j & 15);
 #pragma unroll
     for (int r = 0; r < 16; r++)
-        v[r] = lds[LP(j + 256 * r)];
+        buf[LPR(base, 16 * r)] = v[REV16(r)];
     __syncthreads();
-#pragma unroll
-    for (int r = 1; r < 16; r++) {
-        float2 w = tw2[r];
-        v[r] = cmul(v[r], make_float2(w.x, S * w.y));
-    }
-    dft16<S>(v);
-    float2 o[16];
-#pragma unroll
-    for (int r = 0; r < 16; r++)
-        o[r] = v[OUTSLOT(r)];
-#pragma unroll
-    for (int r = 0; r < 16; r++)
-        v[r] = o[r];
 }
 
-/* Fused correlation for segments of L = 4096 half-bins.  Block id ->
- * (segment, template group); groups is a multiple of 8 so each XCD (block
- * ids are dealt round-robin over the 8 XCDs) touches one residue class of
- * template groups and keeps those templates in its own L2.  The forward
- * FFT of a segment is shared by the group's templates.  The first
- * inter-pass twiddles come from a 2 KiB LDS table (16 distinct values per
- * pass and thread), the second stay in registers: 196 VGPRs, two waves
- * per SIMD. */
-__global__ __launch_bounds__(256) void k_corr4096(const float2 *spec, long long numbins,
-                                                  long long lobin_file, const float2 *T,
-                                                  int nt, int hw, int uselen, long long hb_end,
-                                                  float *plane, int groups, int tpg,
-                                                  long long seg0, long long nsr)
+/* Fused correlation for segments of 4096 half-bins.  The segment's odd
+ * half-bins are zero, so its transform D repeats after 2048 points and the
+ * even and the odd half-bins of D T's inverse transform are two transforms
+ * of 2048 points (k_template_dft): waves 0-1 run the even one, waves 2-3
+ * the odd one (radix 16 and 16, 16 points per thread), and the last,
+ * radix-8, pass gives each thread two adjacent half-bins 8 times, stored
+ * as one float2.  A workgroup keeps D in registers over its group's
+ * templates.
+ *
+ * Bound: FP32 VALU issue.  ~570 vector instructions per thread and
+ * template (196 for the template product and the first radix 16, 192, 144,
+ * 32 for the powers) and ~80 for the stores, against ~760 for one
+ * 4096-point transform with separate twiddle products: 2.0 ms of issue for
+ * the 2^23-sample, zmax 200 search, measured 2.87 ms beside the norms
+ * (3.91 ms before; 2^20 samples, 201 x 31 templates: 10.6 ms, 14.1 ms).
+ * 124 VGPRs and 35 KB of LDS: four workgroups per CU, against two. */
+__global__ __launch_bounds__(256, 4) void k_corr(const float2 *spec, long long numbins,
+                                                 long long lobin_file, const float2 *T, int nt,
+                                                 int hw, int uselen, long long hb_end,
+                                                 float *plane, int groups, int tpg,
+                                                 long long seg0, long long nsr)
 {
-    __shared__ float2 lds[FFT_LDS];
-    __shared__ float2 tw1l[256];
-    const int j = threadIdx.x;
+    __shared__ float2 lds[2 * FFT_LDS];
+    const int tid = threadIdx.x, j = tid & 127;
+    const int odd = __builtin_amdgcn_readfirstlane(tid >> 7);
+    float2 *buf = lds + odd * FFT_LDS;
     /* XCD x (block ids x, x + 8, ...) takes the template groups x, x + 8,
      * ... one after another, each over all nsr segments, so the workgroups
      * resident on an XCD share one group's templates in its L2 (a jerk
@@ -645,55 +734,132 @@ __global__ __launch_bounds__(256) void k_corr4096(const float2 *spec, long long 
     if (t0 >= nt)
         return;
     const int t1 = min(nt, t0 + tpg);
+    /* pass-2 twiddles of the 16 values of j % 16: read from LDS by every
+     * template (8 of 16 apart would cost 16 registers); rows 5 float4 apart
+     * keep 16-byte reads of the 16 rows on distinct banks */
+    __shared__ float4 tw2l[16 * 5];
+    if (tid < 128) {
+        static const int off[8] = {0, 0, 0, 32, 0, 16, 32, 48}, mul[8] = {8, 4, 2, 2, 1, 1, 1, 1};
+        const int m = tid >> 3, k = tid & 7;
+        ((float2 *) (tw2l + 5 * m))[k] = unit_root(mul[k] * m + off[k], 256);
+    }
+    const float4 *tw2 = tw2l + 5 * (j & 15);
+    float2 tw3[4];
     {
-        double s, c;
-        sincospi(2.0 * (double) ((j >> 4) * (j & 15)) / 256.0, &s, &c);
-        tw1l[j] = make_float2((float) c, (float) s);
-    }
-    float2 tw2[16];
-#pragma unroll
-    for (int r = 1; r < 16; r++) {
-        double s, c;
-        sincospi(2.0 * (double) (r * j) / 4096.0, &s, &c);
-        tw2[r] = make_float2((float) c, (float) s);
+        tw3[0] = unit_root(4 * tid, 2048);
+        tw3[1] = unit_root(2 * tid, 2048);
+        tw3[2] = unit_root(tid, 2048);
+        tw3[3] = unit_root(tid + 256, 2048);
     }
 
-    float2 v[16];
-#pragma unroll
-    for (int r = 0; r < 16; r++) {
-        v[r] = make_float2(0.0f, 0.0f);
-        if (!(j & 1)) {
-            long long bin = lobin + ((j + 256 * r) >> 1) - lobin_file;
-            if (bin >= 0 && bin < numbins)
-                v[r] = spec[bin];
-        }
-    }
-    __syncthreads();
-    fft4096<-1>(v, lds, tw1l, tw2);
+    /* D = conj(inverse FFT of the conjugated bins), by both halves */
     float2 D[16];
-#pragma unroll
-    for (int r = 0; r < 16; r++)
-        D[r] = v[r];
-
-    for (int t = t0; t < t1; t++) {
-        const float2 *Tt = T + (size_t) t * 4096;
-#pragma unroll
-        for (int r = 0; r < 16; r++)
-            v[r] = cmul(D[r], Tt[j + 256 * r]);
-        fft4096<1>(v, lds, tw1l, tw2);
+    {
+        float2 v[16];
 #pragma unroll
         for (int r = 0; r < 16; r++) {
-            const int q = j + 256 * r - 2 * hw;
-            const long long hb = seg_hb + q;
-            if (q >= 0 && q < uselen && hb < hb_end) {
-                const float p = __builtin_fmaf(v[r].x, v[r].x, v[r].y * v[r].y);
-                plane[AGPU_PLANE_IDX(t, hb, nt)] = p;
-                /* the first AGPU_HALO half-bins of a tile are repeated in
-                 * the previous tile's halo */
-                if ((hb & (AGPU_TILE - 1)) < AGPU_HALO && hb >= AGPU_TILE)
-                    plane[AGPU_PLANE_IDX(t, hb - AGPU_TILE, nt) + AGPU_TILE] = p;
+            v[r] = make_float2(0.0f, 0.0f);
+            const long long bin = lobin + j + 128 * r - lobin_file;
+            if (bin >= 0 && bin < numbins) {
+                v[r] = spec[bin];
+                v[r].y = -v[r].y;
             }
         }
+#pragma unroll
+        for (int r = 0; r < 8; r++)
+            bfly1(v[r], v[r + 8]);
+        dft16_rest(v);
+        fft2048_mid(v, buf, j, tw2);   /* its first barrier covers tw2l too */
+        float2 u[8];
+#pragma unroll
+        for (int r = 0; r < 8; r++)
+            u[r] = lds[LPR(tid, 256 * r)];
+        dft8_tw(u, tw3);
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < 8; r++)
+            lds[LPR(tid, 256 * r)] = u[REV8(r)];
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+            D[r] = lds[LPR(j, 128 * r)];
+            D[r].y = -D[r].y;
+        }
+    }
+
+    /* this thread's half-bin pairs, 2 tid + 512 k - 2 hw from the segment's
+     * first: byte offsets from the first tile's row, ~0 outside the segment */
+    const long long tile_stride = (long long) nt * AGPU_ROWLEN;
+    const long long tile0 = seg_hb >> AGPU_TILE_LOG2;
+    const int e0 = (int) (seg_hb & (AGPU_TILE - 1));
+    const int lim = (int) min((long long) uselen, hb_end - seg_hb);
+    unsigned off[8];
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+        const int q = 2 * tid + 512 * k - 2 * hw, e = e0 + q;   /* from the tile's start */
+        off[k] = ~0u;
+        if (q >= 0 && q < lim)
+            off[k] = 4u * (unsigned) (e < AGPU_TILE ? e : (int) tile_stride + e - AGPU_TILE);
+    }
+    /* the first AGPU_HALO half-bins of a tile are repeated in the previous
+     * tile's halo: does the segment touch any? */
+    const bool halo = (e0 < AGPU_HALO && tile0 > 0) || e0 + lim > AGPU_TILE;
+    const int eq = e0 + 2 * tid - 2 * hw;
+    float *trow = plane + tile0 * tile_stride + (long long) t0 * AGPU_ROWLEN;
+    float *hrow = trow - tile_stride + AGPU_TILE;   /* the previous tile's halo */
+    const float4 *Tt = (const float4 *) (T + (size_t) t0 * CORR_N + odd * FFT_HALF) + j;
+    for (int t = t0; t < t1; t++) {
+        float2 v[16];
+        /* template product fused with the first radix-2 stage */
+#pragma unroll
+        for (int r = 0; r < 8; r++) {
+            const float4 w = Tt[128 * r];
+            const float2 d = D[r];
+            float2 a = make_float2(__builtin_fmaf(-d.y, w.y, d.x * w.x),
+                                   __builtin_fmaf(d.y, w.x, d.x * w.y));
+            float2 b = D[r + 8];
+            bfly(a, b, make_float2(w.z, w.w));
+            v[r] = a;
+            v[r + 8] = b;
+        }
+        dft16_rest(v);
+        __syncthreads();   /* the previous template's last reads */
+        fft2048_mid(v, buf, j, tw2);
+        float2 u[8], o[8];
+#pragma unroll
+        for (int r = 0; r < 8; r++) {
+            u[r] = lds[LPR(tid, 256 * r)];
+            o[r] = lds[FFT_LDS + LPR(tid, 256 * r)];
+        }
+        dft8_tw(u, tw3);
+        dft8_tw(o, tw3);
+        float2 p[8];
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+            const float2 a = u[REV8(k)], b = o[REV8(k)];
+            p[k] = make_float2(__builtin_fmaf(a.x, a.x, a.y * a.y),
+                               __builtin_fmaf(b.x, b.x, b.y * b.y));
+            if (off[k] != ~0u)
+                *(float2 *) ((char *) trow + off[k]) = p[k];
+        }
+        if (halo) {
+            /* kept out of the loop's invariants: eight more addresses held
+             * over the loop would spill */
+            int e = eq;
+            asm volatile("" : "+v"(e));
+#pragma unroll
+            for (int k = 0; k < 8; k++) {
+                const unsigned b = 4u * (unsigned) (e + 512 * k);
+                if (off[k] != ~0u && e + 512 * k < AGPU_HALO && tile0 > 0)
+                    *(float2 *) ((char *) hrow + b) = p[k];
+                if (off[k] != ~0u && e + 512 * k >= AGPU_TILE &&
+                    e + 512 * k < AGPU_TILE + AGPU_HALO)
+                    *(float2 *) ((char *) trow + b) = p[k];
+            }
+        }
+        trow += AGPU_ROWLEN;
+        hrow += AGPU_ROWLEN;
+        Tt += CORR_N / 2;
     }
 }
 
@@ -1419,8 +1585,8 @@ static int gen_responses(const int *zs, const int *ws, const int *numkern, int n
             AGPU_TRY(hipGetLastError());
         }
         if (d_T) {
-            dim3 g2((L + 255) / 256, nt);
-            hipLaunchKernelGGL(k_template_dft, g2, dim3(256), 0, st, d_resp, d_nk, nkmax, L,
+            dim3 g2(CORR_N / 2 / 256, nt);
+            hipLaunchKernelGGL(k_template_dft, g2, dim3(256), 0, st, d_resp, d_nk, nkmax,
                                (float2 *) d_T);
             AGPU_TRY(hipGetLastError());
         }
@@ -1452,8 +1618,8 @@ cleanup:
 int agpu_gen_templates(const int *zs, const int *ws, const int *numkern, int nt, int L,
                        void *d_T, void *stream)
 {
-    if (nt <= 0 || L <= 0 || nt > 65535 || !d_T)
-        return fail("agpu_gen_templates: bad template count or length");
+    if (nt <= 0 || L != CORR_N || nt > 65535 || !d_T)
+        return fail("agpu_gen_templates: bad template count, or a length other than 4096");
     return gen_responses(zs, ws, numkern, nt, L, d_T, 0, NULL, stream);
 }
 
@@ -1504,9 +1670,9 @@ int agpu_correlate(const void *d_spec, long long numbins, long long lobin_file,
                    float *d_plane, long long ntiles, int groups, long long seg_lo,
                    long long seg_hi, void *stream)
 {
-    if (L != 4096)
+    if (L != CORR_N)
         return fail("agpu_correlate: only L = 4096 is built");
-    if (uselen <= 0 || uselen % 2 || uselen > L - 4 * hw + 1)
+    if (uselen <= 0 || uselen % 2 || uselen > L - 4 * hw + 1 || hb_end % 2)
         return fail("agpu_correlate: uselen must be even and <= L - 4*hw + 1");
     if (groups <= 0 || groups % 8)
         return fail("agpu_correlate: groups must be a positive multiple of 8");
@@ -1523,7 +1689,7 @@ int agpu_correlate(const void *d_spec, long long numbins, long long lobin_file,
     long long nblk = (seg_hi - seg_lo) * groups;
     if (nblk >= (1LL << 24))   /* a dispatch counts work-items in 32 bits */
         return fail("agpu_correlate: grid too large");
-    hipLaunchKernelGGL(k_corr4096, dim3((unsigned) nblk), dim3(256), 0, (hipStream_t) stream,
+    hipLaunchKernelGGL(k_corr, dim3((unsigned) nblk), dim3(256), 0, (hipStream_t) stream,
                        (const float2 *) d_spec, numbins, lobin_file, (const float2 *) d_T, nt,
                        hw, uselen, hb_end, d_plane, groups, tpg, seg_lo, seg_hi - seg_lo);
     AGPU_CHECK(hipGetLastError());
