@@ -15,7 +15,8 @@
  *       (the template loop of src/accel_utils.c:1141-1190).
  *   k_harmsum : harmonic summing with the reference's index rules and
  *       per-block normalisation, and the threshold of search_ffdotpows
- *       (src/accel_utils.c:1261-1452).
+ *       (src/accel_utils.c:1261-1452); k_harmbound : the same hits from
+ *       bounds of the powers, the sums formed only where a bound crosses.
  */
 #include <hip/hip_runtime.h>
 #include <pthread.h>
@@ -662,6 +663,25 @@ __device__ static float2 unit_root(int a, int n)
 
 /* LDS slot of point i: one slot of padding every 16.  LPR(i, r): of point
  * i + r, r a multiple of 16 (an immediate offset from i's slot) */
+/* Stores through a buffer descriptor: a 32-bit byte offset from a base that
+ * all lanes share, and the offset OFF_NONE is out of range, so the hardware
+ * drops that lane's store. */
+#define OFF_NONE 0xffffffffu
+typedef unsigned v2u __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t plane_rsrc(float *p)
+{
+    return __builtin_amdgcn_make_buffer_rsrc(p, 0, (int) 0xfffffff0u, 0x00027000);
+}
+__device__ __forceinline__ void store_pair(__amdgpu_buffer_rsrc_t r, unsigned off, float2 v)
+{
+    const v2u u = {__float_as_uint(v.x), __float_as_uint(v.y)};
+    __builtin_amdgcn_raw_buffer_store_b64(u, r, (int) off, 0, 0);
+}
+__device__ __forceinline__ void store_bound(__amdgpu_buffer_rsrc_t r, unsigned off, unsigned v)
+{
+    __builtin_amdgcn_raw_buffer_store_b16((unsigned short) v, r, (int) off, 0, 0);
+}
+
 #define LP(i) ((i) + ((i) >> 4))
 #define LPR(i, r) (LP(i) + (r) + (r) / 16)
 #define FFT_HALF (CORR_N / 2)
@@ -712,6 +732,7 @@ __device__ __forceinline__ void fft2048_mid(float2 *v, float2 *buf, int j, const
  * the 2^23-sample, zmax 200 search, measured 2.87 ms beside the norms
  * (3.91 ms before; 2^20 samples, 201 x 31 templates: 10.6 ms, 14.1 ms).
  * 124 VGPRs and 35 KB of LDS: four workgroups per CU, against two. */
+template <bool BOUNDS>
 __global__ __launch_bounds__(256, 4) void k_corr(const float2 *spec, long long numbins,
                                                  long long lobin_file, const float2 *T, int nt,
                                                  int hw, int uselen, long long hb_end,
@@ -788,25 +809,42 @@ __global__ __launch_bounds__(256, 4) void k_corr(const float2 *spec, long long n
     }
 
     /* this thread's half-bin pairs, 2 tid + 512 k - 2 hw from the segment's
-     * first: byte offsets from the first tile's row, ~0 outside the segment */
+     * first: byte offsets from the first tile's row */
     const long long tile_stride = (long long) nt * AGPU_ROWLEN;
     const long long tile0 = seg_hb >> AGPU_TILE_LOG2;
     const int e0 = (int) (seg_hb & (AGPU_TILE - 1));
     const int lim = (int) min((long long) uselen, hb_end - seg_hb);
+    const unsigned next = 4u * (unsigned) (tile_stride - AGPU_TILE);   /* the next tile's row */
     unsigned off[8];
 #pragma unroll
     for (int k = 0; k < 8; k++) {
-        const int q = 2 * tid + 512 * k - 2 * hw, e = e0 + q;   /* from the tile's start */
-        off[k] = ~0u;
+        const int q = 2 * tid + 512 * k - 2 * hw, e = e0 + q;   /* e: from the tile's start */
+        off[k] = OFF_NONE;
         if (q >= 0 && q < lim)
-            off[k] = 4u * (unsigned) (e < AGPU_TILE ? e : (int) tile_stride + e - AGPU_TILE);
+            off[k] = 4u * (unsigned) e + (e < AGPU_TILE ? 0u : next);
     }
-    /* the first AGPU_HALO half-bins of a tile are repeated in the previous
-     * tile's halo: does the segment touch any? */
-    const bool halo = (e0 < AGPU_HALO && tile0 > 0) || e0 + lim > AGPU_TILE;
+    /* the first half-bins of a tile (AGPU_HALO of them, or with BOUNDS the
+     * first AGPU_BHALO groups) are repeated behind the previous tile's row:
+     * does the segment touch any? */
+    const int rep = BOUNDS ? AGPU_GROUP * AGPU_BHALO : AGPU_HALO;
+    const bool halo = (e0 < rep && tile0 > 0) || e0 + lim > AGPU_TILE;
     const int eq = e0 + 2 * tid - 2 * hw;
+    /* BOUNDS: lanes 2 i and 2 i + 1 hold one group of AGPU_GROUP half-bins
+     * for each k; the even lane stores the bound for k = 2 m, the odd one
+     * for k = 2 m + 1 */
+    const int eg = e0 + 2 * (tid & ~1) + 512 * (tid & 1) - 2 * hw;
+    unsigned goff[4];
+#pragma unroll
+    for (int m = 0; m < 4; m++) {
+        const int e = eg + 1024 * m, q = e - e0;
+        goff[m] = OFF_NONE;
+        if (BOUNDS && q >= 0 && q < lim)
+            goff[m] = e < AGPU_TILE
+                          ? 4u * AGPU_TILE + 2u * (unsigned) (e / AGPU_GROUP)
+                          : 4u * (unsigned) tile_stride + 4u * AGPU_TILE +
+                                2u * (unsigned) ((e - AGPU_TILE) / AGPU_GROUP);
+    }
     float *trow = plane + tile0 * tile_stride + (long long) t0 * AGPU_ROWLEN;
-    float *hrow = trow - tile_stride + AGPU_TILE;   /* the previous tile's halo */
     const float4 *Tt = (const float4 *) (T + (size_t) t0 * CORR_N + odd * FFT_HALF) + j;
     for (int t = t0; t < t1; t++) {
         float2 v[16];
@@ -833,32 +871,60 @@ __global__ __launch_bounds__(256, 4) void k_corr(const float2 *spec, long long n
         }
         dft8_tw(u, tw3);
         dft8_tw(o, tw3);
+        const __amdgpu_buffer_rsrc_t row = plane_rsrc(trow);
+        /* behind the previous tile's row (no tile before the first: nothing
+         * is stored there, every offset is OFF_NONE) */
+        const __amdgpu_buffer_rsrc_t prev =
+            plane_rsrc(tile0 > 0 ? trow - tile_stride + AGPU_TILE : trow);
         float2 p[8];
 #pragma unroll
         for (int k = 0; k < 8; k++) {
             const float2 a = u[REV8(k)], b = o[REV8(k)];
             p[k] = make_float2(__builtin_fmaf(a.x, a.x, a.y * a.y),
                                __builtin_fmaf(b.x, b.x, b.y * b.y));
-            if (off[k] != ~0u)
-                *(float2 *) ((char *) trow + off[k]) = p[k];
+            store_pair(row, off[k], p[k]);
         }
-        if (halo) {
-            /* kept out of the loop's invariants: eight more addresses held
-             * over the loop would spill */
+        if (BOUNDS) {
+            /* the group's largest power rounded up to 16 bits: an upper bound
+             * that the harmonic sum looks at before it reads the powers.  Bit
+             * patterns, which order like the powers: a NaN stays one */
+            int e = eg;
+            asm volatile("" : "+v"(e));   /* see below */
+#pragma unroll
+            for (int m = 0; m < 4; m++) {
+                unsigned w[2];
+#pragma unroll
+                for (int h = 0; h < 2; h++) {
+                    const unsigned x = max(__float_as_uint(p[2 * m + h].x),
+                                           __float_as_uint(p[2 * m + h].y));
+                    w[h] = max(x, (unsigned) __builtin_amdgcn_update_dpp(
+                                      0, (int) x, 0xb1 /* lanes 1,0,3,2 */, 0xf, 0xf, true));
+                }
+                const unsigned bnd = ((tid & 1 ? w[1] : w[0]) + 0xffffu) >> 16;
+                store_bound(row, goff[m], bnd);
+                if (halo) {
+                    const unsigned g = (unsigned) (e + 1024 * m) / AGPU_GROUP;
+                    const bool ok = goff[m] != OFF_NONE;
+                    store_bound(prev, ok && tile0 > 0 && g < AGPU_BHALO ? 2 * (g + AGPU_TILE / AGPU_GROUP)
+                                                           : OFF_NONE, bnd);
+                    store_bound(row, ok && g - AGPU_TILE / AGPU_GROUP < AGPU_BHALO
+                                         ? 4u * AGPU_TILE + 2 * g : OFF_NONE, bnd);
+                }
+            }
+        } else if (halo) {
+            /* kept out of the loop's invariants: more addresses held over the
+             * loop would spill */
             int e = eq;
             asm volatile("" : "+v"(e));
 #pragma unroll
             for (int k = 0; k < 8; k++) {
-                const unsigned b = 4u * (unsigned) (e + 512 * k);
-                if (off[k] != ~0u && e + 512 * k < AGPU_HALO && tile0 > 0)
-                    *(float2 *) ((char *) hrow + b) = p[k];
-                if (off[k] != ~0u && e + 512 * k >= AGPU_TILE &&
-                    e + 512 * k < AGPU_TILE + AGPU_HALO)
-                    *(float2 *) ((char *) trow + b) = p[k];
+                const unsigned x = (unsigned) (e + 512 * k);
+                const bool ok = off[k] != OFF_NONE;
+                store_pair(prev, ok && tile0 > 0 && x < AGPU_HALO ? 4 * x : OFF_NONE, p[k]);
+                store_pair(row, ok && x - AGPU_TILE < AGPU_HALO ? 4 * x : OFF_NONE, p[k]);
             }
         }
         trow += AGPU_ROWLEN;
-        hrow += AGPU_ROWLEN;
         Tt += CORR_N / 2;
     }
 }
@@ -874,6 +940,10 @@ __global__ __launch_bounds__(256, 4) void k_corr(const float2 *spec, long long n
 #define HS_CT AGPU_HS_CT
 #define HS_CPT 4
 #define HS_CHUNK (HS_TPB * HS_CPT)
+#define HB_CHUNK (64 * AGPU_GROUP)   /* half-bins per workgroup of k_harmbound */
+#define HB_MINROWS 16                /* z rows, cells below which k_harmsum is faster */
+#define HB_MINCELLS (1LL << 23)
+#define HB_ROWS 64                   /* z rows per workgroup of k_harmbound at most */
 
 __device__ __forceinline__ void emit_hit(const agpu_harmsum_args &a, int b, int s, int wi,
                                          int zi, int ii, float p)
@@ -1218,6 +1288,366 @@ __global__ __launch_bounds__(HS_TPB) void k_harmsum(agpu_harmsum_args a, int c_l
     }
 #undef HS_STAGE
 #undef HS_EMIT
+}
+
+/* ---- the harmonic sum over bounds ---- */
+
+/* Largest norm^2 that the cells of each 256-half-bin chunk meet, per
+ * fraction ([chunk][32], fundamental first), raised by 2^-18: the bounds'
+ * multiply-adds round differently than the cells' products and sums (16
+ * roundings of 2^-24 each at most).  A NaN norm is skipped (its cells cross
+ * no threshold) unless all are NaN. */
+template <int MODE>
+__global__ void k_bound_norms(agpu_harmsum_args a, int c0, int nc, long long hb_end, float *nb)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    const int c = i >> 5, f = i & 31;
+    if (c >= nc || f > a.nfrac)
+        return;
+    const int hb = (c0 + c) * HB_CHUNK;
+    const int rh0 = (int) a.rh0, cu = a.corr_uselen;
+    float m;
+    if (MODE == HS_INMEM) {
+        /* f = 2^(s-1) + (k-1)/2 for fraction k / 2^s; 0 is the fundamental */
+        const int s = f ? 32 - __clz(f) : 0, k = f ? 2 * (f - (1 << (s - 1))) + 1 : 1;
+        const int end = (int) hb_end - 1;
+        const int lo = min(hs_round<HS_INMEM>(hb, k, s), end);
+        const int hi = min(hs_round<HS_INMEM>(hb + HB_CHUNK - 1, k, s), end);
+        /* a span shorter than a block meets at most two blocks on either
+         * side of rh0, where the pre-population ends */
+        m = fmaxf(a.nsq_hb[lo], a.nsq_hb[hi]);
+        if (lo < rh0 && rh0 <= hi)
+            m = fmaxf(m, fmaxf(a.nsq_hb[rh0 - 1], a.nsq_hb[rh0]));
+    } else {
+        const int nfr = a.nfrac + 1;
+        const int b0 = min(max(hb - rh0, 0) / cu, a.nblocks - 1);
+        const int b1 = min(max(hb + HB_CHUNK - 1 - rh0, 0) / cu, a.nblocks - 1);
+        m = fmaxf(a.nsq[(size_t) b0 * nfr + f], a.nsq[(size_t) b1 * nfr + f]);
+    }
+    nb[(size_t) c * 32 + f] = m + m * 0x1p-18f;
+}
+
+/* Exact sums of 64 cells, lane l at fundamental half-bin hb + l, of every
+ * z row z0 + i with bit i set in todo (not 0), straight from the raw plane:
+ * the terms and their order are k_harmsum's.  The lanes of a fraction lie
+ * in one tile or the next, so their offsets from the first lane's tile-row
+ * fit 32 bits; offsets and norms serve all rows. */
+template <int NSTAGES, int MODE>
+__device__ __forceinline__ void hb_cells(const agpu_harmsum_args &a, long long tile_stride, int hb,
+                                         int lane, int wi, int z0, unsigned long long todo)
+{
+#pragma clang fp contract(off)
+    constexpr int NF = 1 << (NSTAGES - 1);
+    const int rh = hb + lane, c = rh - (int) a.rh0;
+    const bool in = c >= 0 && c < a.nblocks * a.corr_uselen;
+    const int b = in ? c / a.corr_uselen : 0;
+    const unsigned next = 4u * (unsigned) (tile_stride - AGPU_TILE);
+    const char *base[NF];
+    unsigned off[NF];
+    float nn[NF];
+#pragma unroll
+    for (int f = 0; f < NF; f++) {
+        const int S = f ? 32 - __builtin_clz(f) : 0, k = f ? 2 * (f - (1 << S >> 1)) + 1 : 1;
+        const int first = S ? hs_round<MODE>(hb, k, S) : hb;
+        const int rs = S ? hs_round<MODE>(rh, k, S) : rh;
+        const int t0 = first & ~(AGPU_TILE - 1);
+        const unsigned x = (unsigned) (rs - t0);
+        base[f] = (const char *) (a.plane + (t0 >> AGPU_TILE_LOG2) * tile_stride);
+        off[f] = 4u * x + (x < AGPU_TILE ? 0u : next);
+        nn[f] = MODE == HS_INMEM ? a.nsq_hb[rs] : a.nsq[(size_t) b * NF + f];
+    }
+    while (todo) {   /* two rows' loads in flight */
+        int zi[2];
+        zi[0] = z0 + (int) __ffsll(todo) - 1;
+        todo &= todo - 1;
+        const bool pair = todo != 0;
+        zi[1] = pair ? z0 + (int) __ffsll(todo) - 1 : zi[0];
+        todo &= todo - 1;   /* 0 stays 0 */
+        float val[2][NF];
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const unsigned *rt = a.row_tab + (size_t) (wi * a.numz + zi[h]) * HS_RT;
+#pragma unroll
+            for (int f = 0; f < NF; f++)
+                val[h][f] = *(const float *) (base[f] +
+                                              4 * (size_t) rt[f ? HS_RT_SUB + f - 1 : HS_RT_ROW] +
+                                              off[f]);
+        }
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            float acc[NSTAGES];
+            acc[0] = val[h][0] * nn[0];
+            bool hit = acc[0] > a.powcut[0];
+#pragma unroll
+            for (int S = 1; S < NSTAGES; S++) {
+                acc[S] = acc[S - 1];
+#pragma unroll
+                for (int f = 1 << (S - 1); f < (1 << S); f++)
+                    acc[S] = acc[S] + val[h][f] * nn[f];
+                hit |= acc[S] > a.powcut[S];
+            }
+            if (in && hit && (h == 0 || pair))
+#pragma unroll
+                for (int S = 0; S < NSTAGES; S++)
+                    if (acc[S] > a.powcut[S])
+                        emit_hit(a, b, S, wi, zi[h], c - b * a.corr_uselen, acc[S]);
+        }
+    }
+}
+
+/* ---- LDS tiles of the bounds ----
+ * A workgroup looks through HB_CHUNK half-bins (64 groups) of up to HB_ROWS
+ * consecutive z rows.  For fraction k / 2^s they meet 64 k / 2^s + 1 groups
+ * (32 k / 2^s + 1 dwords of two, an odd stride) of at most
+ * (HB_ROWS - 1) k / 2^s + 3 z rows: the map rounds k z / 2^s half away from
+ * zero, so the ends move apart by less than two rows. */
+__host__ __device__ constexpr int hb_dw(int k, int s) { return (32 * k >> s) + 1; }
+__host__ __device__ constexpr int hb_nr(int k, int s)
+{
+    return s ? ((HB_ROWS - 1) * k >> s) + 3 : HB_ROWS;
+}
+/* lanes per row of a load: the power of two that holds the dwords */
+__host__ __device__ constexpr int hb_lpr(int k, int s)
+{
+    int n = 1;
+    while (n < (s ? hb_dw(k, s) : 32))
+        n *= 2;
+    return n;
+}
+__host__ __device__ constexpr int hb_loads(int k, int s)
+{
+    const int rpp = 256 / hb_lpr(k, s);
+    return (hb_nr(k, s) + rpp - 1) / rpp;
+}
+/* dwords of the tiles of stages s0..s1 before fraction (k, s) */
+__host__ __device__ constexpr int hb_base(int s0, int k, int s)
+{
+    int n = 0;
+    for (int t = s0; t <= s; t++)
+        for (int i = 1; i < (1 << t) + (t == 0); i += 2)
+            if (t < s || i < k)
+                n += hb_dw(i, t) * hb_nr(i, t);
+    return n;
+}
+__host__ __device__ constexpr int hb_size(int s0, int s1) { return hb_base(s0, (1 << s1) + 1, s1); }
+__host__ __device__ constexpr int hb_lds(int nstages)
+{
+    return hs_max(hb_size(0, nstages < 4 ? nstages - 1 : 3), nstages > 4 ? hb_size(4, 4) : 0);
+}
+__host__ __device__ constexpr int hb_nloads(int s0, int s1)
+{
+    int n = 0;
+    for (int t = s0; t <= s1; t++)
+        for (int i = 1; i < (1 << t) + (t == 0); i += 2)
+            n += hb_loads(i, t);
+    return n;
+}
+static_assert(hb_dw(15, 4) <= 32 && 2 * (AGPU_TILE / AGPU_GROUP + AGPU_BHALO) == 4 * AGPU_HALO &&
+                  AGPU_BHALO >= 64 + 2,
+              "a chunk's bounds lie in one tile-row and its replica");
+
+/* The workgroup's loads of fraction k / 2^s into registers: thread t takes
+ * dword t % lpr of row t / lpr (and 256 / lpr rows on). */
+template <int K, int S>
+__device__ __forceinline__ void hb_load(const agpu_harmsum_args &a, unsigned *v, int g0,
+                                        long long tile_stride, int wi, int z0, int z1)
+{
+    constexpr int LPR = hb_lpr(K, S), RPP = 256 / LPR, F = S ? (1 << S >> 1) + (K - 1) / 2 : 0;
+    const int J = g0 * K >> S;   /* exact: g0 is a multiple of 64 */
+    const int zf = S ? a.zmap[(F - 1) * a.numz + z0] : z0;
+    const int nr = (S ? a.zmap[(F - 1) * a.numz + z1 - 1] : z1 - 1) - zf + 1;
+    const int wf = S ? a.wmap[(F - 1) * a.numw + wi] : wi;
+    const char *base = (const char *) (a.plane +
+                                       (long long) (J >> (AGPU_TILE_LOG2 - AGPU_GROUP_LOG2)) *
+                                           tile_stride +
+                                       ((long long) wf * a.numz + zf) * AGPU_ROWLEN + AGPU_TILE) +
+                       2 * (J & (AGPU_TILE / AGPU_GROUP - 1));
+    const int dw = threadIdx.x % LPR, row = threadIdx.x / LPR;
+    const unsigned off = (unsigned) (row * 4 * AGPU_ROWLEN + 4 * dw);
+#pragma unroll
+    for (int u = 0; u < hb_loads(K, S); u++) {
+        v[u] = 0;
+        if (row + u * RPP < nr && (S == 0 || dw < hb_dw(K, S)))
+            v[u] = *(const unsigned *) (base + (off + (unsigned) (u * RPP * 4 * AGPU_ROWLEN)));
+    }
+}
+
+template <int K, int S>
+__device__ __forceinline__ void hb_store(unsigned *lds, const unsigned *v)
+{
+    constexpr int LPR = hb_lpr(K, S), RPP = 256 / LPR;
+    const int dw = threadIdx.x % LPR, row = threadIdx.x / LPR;
+#pragma unroll
+    for (int u = 0; u < hb_loads(K, S); u++)
+        if (row + u * RPP < hb_nr(K, S) && (S == 0 || dw < hb_dw(K, S)))
+            lds[(row + u * RPP) * hb_dw(K, S) + dw] = v[u];
+}
+
+/* Adds fraction k / 2^s to the sums of this wave's 16 groups of this lane's
+ * row.  p: the row's dwords from the wave's first group on (ODD: from the
+ * group before it).  Which groups a sum meets is known at compile time. */
+template <int K, int S, bool ODD>
+__device__ __forceinline__ void hb_add(float *acc, const unsigned *p, float nn)
+{
+    constexpr int N = ((63 * K + (1 << S >> 1)) >> (S + AGPU_GROUP_LOG2)) + 1;   /* groups met */
+    unsigned w[(N + 2) / 2], g[N];
+#pragma unroll
+    for (int i = 0; i < (N + ODD + 1) / 2; i++)
+        w[i] = p[i];
+#pragma unroll
+    for (int j = 0; j < N; j++)   /* the upper group's low half only raises it */
+        g[j] = (j + ODD) & 1 ? w[(j + ODD) / 2] : w[(j + ODD) / 2] << 16;
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+        const int j0 = (AGPU_GROUP * i * K) >> (S + AGPU_GROUP_LOG2);
+        const int j1 = ((AGPU_GROUP * i + AGPU_GROUP - 1) * K + (1 << S >> 1)) >>
+                       (S + AGPU_GROUP_LOG2);
+        /* as integers: powers order like their bits, and an infinite or NaN
+         * bound stays one */
+        const unsigned m = j1 == j0 ? g[j0] : max(g[j0], g[j1]);
+        acc[i] = S ? __builtin_fmaf(__uint_as_float(m), nn, acc[i]) : __uint_as_float(m) * nn;
+    }
+}
+
+/* any of the 16 sums above the threshold, or NaN */
+__device__ __forceinline__ bool hb_over(const float *acc, float cut)
+{
+    unsigned m = __float_as_uint(acc[0]);
+#pragma unroll
+    for (int i = 1; i < 16; i++)
+        m = max(m, __float_as_uint(acc[i]));
+    return !(__uint_as_float(m) <= cut);
+}
+
+/* stage by stage, the fractions of a stage in order */
+template <int K, int S>
+__device__ __forceinline__ void hb_load_stage(const agpu_harmsum_args &a, unsigned *v, int g0,
+                                              long long tile_stride, int wi, int z0, int z1)
+{
+    hb_load<K, S>(a, v, g0, tile_stride, wi, z0, z1);
+    if constexpr (K + 2 < (1 << S))
+        hb_load_stage<K + 2, S>(a, v + hb_loads(K, S), g0, tile_stride, wi, z0, z1);
+}
+template <int K, int S>
+__device__ __forceinline__ void hb_store_stage(unsigned *lds, const unsigned *v)
+{
+    hb_store<K, S>(lds, v);
+    if constexpr (K + 2 < (1 << S))
+        hb_store_stage<K + 2, S>(lds + hb_dw(K, S) * hb_nr(K, S), v + hb_loads(K, S));
+}
+template <int K, int S, bool ODD>
+__device__ __forceinline__ void hb_add_stage(const agpu_harmsum_args &a, float *acc,
+                                             const unsigned *lds, const float *np, int z0, int z,
+                                             int wv)
+{
+    constexpr int F = (1 << S >> 1) + (K - 1) / 2;
+    const int zs = a.zmap[(F - 1) * a.numz + z] - a.zmap[(F - 1) * a.numz + z0];
+    hb_add<K, S, ODD>(acc, lds + zs * hb_dw(K, S) + (wv * (16 * K >> S)) / 2, np[F]);
+    if constexpr (K + 2 < (1 << S))
+        hb_add_stage<K + 2, S, ODD>(a, acc, lds + hb_dw(K, S) * hb_nr(K, S), np, z0, z, wv);
+}
+
+/* The harmonic sum and threshold by bounds.  A workgroup takes 256
+ * fundamental half-bins (64 groups of 4; a wave 16 groups) of up to 64
+ * consecutive z rows (a lane one row).  Each lane sums, in place of the
+ * powers, the largest power of the one or two groups that a group's cells
+ * meet in every sub-harmonic (the 16-bit bounds that k_corr<true> wrote,
+ * rounded up) times the largest norm: no sum of the group's cells exceeds
+ * that at any stage.  Only where it exceeds the stage's threshold (or is
+ * NaN) are the 64 cells around it summed exactly, from the raw plane.  Hits
+ * are those of k_harmsum bit for bit: a cell that crosses is never skipped,
+ * and every emitted sum is formed from the same terms in the same order.
+ *
+ * Lanes along z share sub-harmonic rows, groups along r share sub-harmonic
+ * groups, so each bound is read once into LDS per workgroup ((k / H)^2 of
+ * the fundamental's bytes per fraction), and which groups a sum meets is
+ * the same for every row and chunk: the inner loop is LDS reads, maxima and
+ * multiply-adds without any index arithmetic.
+ *
+ * 2^23 samples, zmax 200, 16 harmonics: 2.1 ms against k_harmsum's 7.4 (1/8
+ * of its 39 GB; 1.3 % of the 64-cell runs summed exactly); 2^20, 201 x 31
+ * templates, 8 harmonics: 3.1 ms against 14.4.  Bound: vector and scalar
+ * issue (1.1 ms of it) and the latency of the two load-store-sum phases at
+ * four waves per SIMD. */
+template <int NSTAGES, int MODE>
+__global__ __launch_bounds__(256) void k_harmbound(agpu_harmsum_args a, const float *nb,
+                                                   int chunks, int zblocks, int zrows)
+{
+    __shared__ unsigned lds[hb_lds(NSTAGES)];
+    const int lane = threadIdx.x & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    /* all rows of a chunk run on one XCD (block ids are dealt round-robin to
+     * the 8), so that row blocks which share sub-harmonic rows find them in
+     * its L2 */
+    const int rb = zblocks * a.numw;
+    const int xcd = blockIdx.x & 7, local = blockIdx.x >> 3;
+    const int c = (local / rb) * 8 + xcd;        /* chunk, from the one of the first cell */
+    const int wi = (local % rb) / zblocks, z0 = (local % rb) % zblocks * zrows;
+    const int z1 = min(a.numz, z0 + zrows);
+    if (c >= chunks)
+        return;
+    const int hb = ((int) a.rh0 / HB_CHUNK + c) * HB_CHUNK, g0 = hb / AGPU_GROUP;
+    const long long tile_stride = (long long) a.numz * a.numw * AGPU_ROWLEN;
+    const float *np = nb + (size_t) c * 32;
+    constexpr int LAST = NSTAGES < 4 ? NSTAGES - 1 : 3;
+    {
+        unsigned v[hb_nloads(0, LAST)];
+        hb_load<1, 0>(a, v, g0, tile_stride, wi, z0, z1);
+        if constexpr (NSTAGES > 1)
+            hb_load_stage<1, 1>(a, v + hb_nloads(0, 0), g0, tile_stride, wi, z0, z1);
+        if constexpr (NSTAGES > 2)
+            hb_load_stage<1, 2>(a, v + hb_nloads(0, 1), g0, tile_stride, wi, z0, z1);
+        if constexpr (NSTAGES > 3)
+            hb_load_stage<1, 3>(a, v + hb_nloads(0, 2), g0, tile_stride, wi, z0, z1);
+        hb_store<1, 0>(lds, v);
+        if constexpr (NSTAGES > 1)
+            hb_store_stage<1, 1>(lds + hb_base(0, 1, 1), v + hb_nloads(0, 0));
+        if constexpr (NSTAGES > 2)
+            hb_store_stage<1, 2>(lds + hb_base(0, 1, 2), v + hb_nloads(0, 1));
+        if constexpr (NSTAGES > 3)
+            hb_store_stage<1, 3>(lds + hb_base(0, 1, 3), v + hb_nloads(0, 2));
+    }
+    unsigned v4[NSTAGES > 4 ? hb_nloads(4, 4) : 1];
+    if constexpr (NSTAGES > 4)   /* in flight while the stages before are summed */
+        hb_load_stage<1, 4>(a, v4, g0, tile_stride, wi, z0, z1);
+    __syncthreads();
+    const int z = min(z0 + lane, z1 - 1);
+    float acc[16];
+    hb_add<1, 0, false>(acc, lds + (z - z0) * hb_dw(1, 0) + wv * 8, np[0]);
+    bool over = hb_over(acc, a.powcut[0]);
+    if constexpr (NSTAGES > 1) {
+        hb_add_stage<1, 1, false>(a, acc, lds + hb_base(0, 1, 1), np, z0, z, wv);
+        over |= hb_over(acc, a.powcut[1]);
+    }
+    if constexpr (NSTAGES > 2) {
+        hb_add_stage<1, 2, false>(a, acc, lds + hb_base(0, 1, 2), np, z0, z, wv);
+        over |= hb_over(acc, a.powcut[2]);
+    }
+    if constexpr (NSTAGES > 3) {
+        hb_add_stage<1, 3, false>(a, acc, lds + hb_base(0, 1, 3), np, z0, z, wv);
+        over |= hb_over(acc, a.powcut[3]);
+    }
+    if constexpr (NSTAGES > 4) {
+        __syncthreads();
+        hb_store_stage<1, 4>(lds, v4);
+        __syncthreads();
+        /* k groups per wave: an odd wave starts on an odd group */
+        if (wv & 1)
+            hb_add_stage<1, 4, true>(a, acc, lds, np, z0, z, wv);
+        else
+            hb_add_stage<1, 4, false>(a, acc, lds, np, z0, z, wv);
+        over |= hb_over(acc, a.powcut[4]);
+    }
+    const unsigned long long todo = __ballot(over && z0 + lane < z1);
+    if (todo)
+        hb_cells<NSTAGES, MODE>(a, tile_stride, hb + 64 * wv, lane, wi, z0, todo);
+}
+
+/* z rows per workgroup: numz in equal blocks of at most HB_ROWS */
+static int hb_zrows(int numz)
+{
+    const int n = (numz + HB_ROWS - 1) / HB_ROWS;
+    return (numz + n - 1) / n;
 }
 
 /* First half-bin of a chunk's span for fraction k / 2^s.  HS_FRAC starts
@@ -1668,7 +2098,7 @@ int agpu_block_norm1(const void *d_spec, long long numbins, long long lobin_file
 int agpu_correlate(const void *d_spec, long long numbins, long long lobin_file,
                    const void *d_T, int nt, int L, int hw, int uselen, long long hb_end,
                    float *d_plane, long long ntiles, int groups, long long seg_lo,
-                   long long seg_hi, void *stream)
+                   long long seg_hi, int bounds, void *stream)
 {
     if (L != CORR_N)
         return fail("agpu_correlate: only L = 4096 is built");
@@ -1689,9 +2119,17 @@ int agpu_correlate(const void *d_spec, long long numbins, long long lobin_file,
     long long nblk = (seg_hi - seg_lo) * groups;
     if (nblk >= (1LL << 24))   /* a dispatch counts work-items in 32 bits */
         return fail("agpu_correlate: grid too large");
-    hipLaunchKernelGGL(k_corr, dim3((unsigned) nblk), dim3(256), 0, (hipStream_t) stream,
-                       (const float2 *) d_spec, numbins, lobin_file, (const float2 *) d_T, nt,
-                       hw, uselen, hb_end, d_plane, groups, tpg, seg_lo, seg_hi - seg_lo);
+    if (bounds && (uselen % AGPU_GROUP || hw % 2))
+        return fail("agpu_correlate: bounds need segments of whole groups");
+    if (bounds)
+        hipLaunchKernelGGL(k_corr<true>, dim3((unsigned) nblk), dim3(256), 0, (hipStream_t) stream,
+                           (const float2 *) d_spec, numbins, lobin_file, (const float2 *) d_T, nt,
+                           hw, uselen, hb_end, d_plane, groups, tpg, seg_lo, seg_hi - seg_lo);
+    else
+        hipLaunchKernelGGL(k_corr<false>, dim3((unsigned) nblk), dim3(256), 0,
+                           (hipStream_t) stream, (const float2 *) d_spec, numbins, lobin_file,
+                           (const float2 *) d_T, nt, hw, uselen, hb_end, d_plane, groups, tpg,
+                           seg_lo, seg_hi - seg_lo);
     AGPU_CHECK(hipGetLastError());
     return 0;
 }
@@ -1769,6 +2207,119 @@ int agpu_harmsum(const agpu_harmsum_args *a, long long c_lo, long long c_hi, voi
         HS_CASE(6)
     }
 #undef HS_CASE
+    AGPU_CHECK(hipGetLastError());
+    return 0;
+}
+
+/* Bounds pay
+ *  - while few cells pass them: on whitened noise the bound of a sum of H
+ *    powers is 2.13 H on average (the largest of 4 half-bins, or of 4 and 4)
+ *    with a spread of 1.3 sqrt(H); with a threshold 2.4 spreads up a tenth
+ *    of the 64-cell runs are summed exactly.  16 harmonics, 2^18 samples,
+ *    zmax 100 (3.0 sqrt(H) up): 130 us against k_harmsum's 118; 2^19, zmax
+ *    100 (3.3): 151 against 219; 2^21, zmax 100 (3.8): 341 against 1100;
+ *  - with rows for the lanes and workgroups for the device: 8 harmonics,
+ *    2^21 samples, 5 rows 58 us against 37, 11 rows 60 against 62, 21 rows
+ *    62 against 107; 21 rows of 2^18 half-bins 28 against 24, of 2^19 31
+ *    against 36, 51 rows of 2^18 34 against 40. */
+int agpu_harmbound_pays(int nstages, const float *powcut, int corr_uselen, int numz, int numw,
+                        long long numhb, int nfrac, const int *zmap)
+{
+    if (nstages < 1 || nstages > 5 || corr_uselen < HS_CHUNK / 2 || numz < HB_MINROWS ||
+        (long long) numz * numw * numhb < HB_MINCELLS)
+        return 0;
+    for (int s = 0; s < nstages; s++) {
+        const double H = 1 << s;
+        if (!(powcut[s] >= 2.13 * H + 3.1 * sqrt(H)))
+            return 0;
+    }
+    /* the LDS tiles hold every row block's sub-harmonic rows */
+    const int zrows = hb_zrows(numz);
+    for (int f = 1; f <= nfrac; f++) {
+        const int s = 32 - __builtin_clz(f), k = 2 * (f - (1 << (s - 1))) + 1;
+        for (int z0 = 0; z0 < numz; z0 += zrows) {
+            const int z1 = z0 + zrows < numz ? z0 + zrows : numz;
+            const int *m = zmap + (size_t) (f - 1) * numz;
+            for (int z = z0 + 1; z < z1; z++)
+                if (m[z] < m[z - 1])
+                    return 0;
+            if (m[z1 - 1] - m[z0] + 1 > hb_nr(k, s))
+                return 0;
+        }
+    }
+    return 1;
+}
+
+long long agpu_harmbound_chunks(const agpu_harmsum_args *a)
+{
+    const long long ncell = (long long) a->nblocks * a->corr_uselen;
+    return ncell > 0 ? (a->rh0 + ncell - 1) / HB_CHUNK - a->rh0 / HB_CHUNK + 1 : 0;
+}
+
+int agpu_bound_norms(const agpu_harmsum_args *a, long long hb_end, float *d_nb, void *stream)
+{
+    const long long nc = agpu_harmbound_chunks(a);
+    if (nc <= 0)
+        return 0;
+    const int c0 = (int) (a->rh0 / HB_CHUNK);
+    const dim3 grid((unsigned) ((nc * 32 + 255) / 256));
+    if (a->inmem)
+        hipLaunchKernelGGL(k_bound_norms<HS_INMEM>, grid, dim3(256), 0, (hipStream_t) stream, *a,
+                           c0, (int) nc, hb_end, d_nb);
+    else
+        hipLaunchKernelGGL(k_bound_norms<HS_STD>, grid, dim3(256), 0, (hipStream_t) stream, *a, c0,
+                           (int) nc, hb_end, d_nb);
+    AGPU_CHECK(hipGetLastError());
+    return 0;
+}
+
+int agpu_harmbound(const agpu_harmsum_args *a, const float *d_nb, void *stream)
+{
+    const long long ncell = (long long) a->nblocks * a->corr_uselen;
+    if (ncell <= 0)
+        return 0;
+    if (a->nstages < 1 || a->nstages > 5 || a->nfrac + 1 != 1 << (a->nstages - 1) || a->bstart ||
+        a->rh_off)
+        return fail("agpu_harmbound: 1..5 stages, blocks that start on whole bins");
+    if (a->corr_uselen < HS_CHUNK / 2)
+        return fail("agpu_harmbound: corr_uselen below 512 half-bins");
+    if (a->inmem && !a->nsq_hb)
+        return fail("agpu_harmbound: in-memory path needs the per-half-bin norm table");
+    const long long rh_end = a->rh0 + ncell;
+    if (a->ntiles < ((rh_end - 1) >> AGPU_TILE_LOG2) + 2 || a->ntiles * AGPU_TILE > 0x7fffffffLL)
+        return fail("agpu_harmbound: plane tiles must pad the half-bin range by one tile "
+                    "and stay below 2^31 half-bins");
+    if ((rh_end + HS_CHUNK) * (long long) ((1 << (a->nstages - 1)) - 1) > 0x7fffffffLL)
+        return fail("agpu_harmbound: spectrum too long for 32-bit sub-harmonic indices "
+                    "(half-bins x highest harmonic must stay below 2^31)");
+    if (!a->row_tab || (a->nfrac && (!a->zmap || !a->wmap)))
+        return fail("agpu_harmbound: row tables missing");
+    if ((long long) a->numz * a->numw * AGPU_ROWLEN > 0x3fffffffLL)
+        return fail("agpu_harmbound: too many rows for 32-bit row offsets");
+    const int zrows = hb_zrows(a->numz), zblocks = (a->numz + zrows - 1) / zrows;
+    const long long nc = agpu_harmbound_chunks(a);
+    const long long nblk = (nc + 7) / 8 * 8 * zblocks * a->numw;
+    if (nblk >= (1LL << 24))   /* a dispatch counts work-items in 32 bits */
+        return fail("agpu_harmbound: grid too large");
+    const dim3 grid((unsigned) nblk);
+    hipStream_t st = (hipStream_t) stream;
+#define HB_CASE(NS)                                                                          \
+    case NS:                                                                                 \
+        if (a->inmem)                                                                        \
+            hipLaunchKernelGGL((k_harmbound<NS, HS_INMEM>), grid, dim3(256), 0, st, *a, d_nb, \
+                               (int) nc, zblocks, zrows);                                    \
+        else                                                                                 \
+            hipLaunchKernelGGL((k_harmbound<NS, HS_STD>), grid, dim3(256), 0, st, *a, d_nb,   \
+                               (int) nc, zblocks, zrows);                                    \
+        break;
+    switch (a->nstages) {
+        HB_CASE(1)
+        HB_CASE(2)
+        HB_CASE(3)
+        HB_CASE(4)
+        HB_CASE(5)
+    }
+#undef HB_CASE
     AGPU_CHECK(hipGetLastError());
     return 0;
 }

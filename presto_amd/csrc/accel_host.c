@@ -322,6 +322,8 @@ struct accel_search {
     double *d_norm;
     float *d_nsq;
     float *d_nsq_hb;      /* in-memory path: per-half-bin norm^2 */
+    int bounds;           /* harmonic sum by group bounds (agpu_harmbound) */
+    float *d_nb;          /* its norm table */
     int *d_zmap, *d_wmap;
     unsigned *d_rowtab;   /* harmonic-sum address tables (agpu.h) */
     long long *d_cbase;
@@ -623,6 +625,37 @@ static int photon_norms(accel_search *s)
     return 0;
 }
 
+static void fill_harmsum_args(const accel_search *s, agpu_harmsum_args *a)
+{
+    const accel_geom *g = &s->g;
+    memset(a, 0, sizeof(*a));
+    a->plane = s->d_plane;
+    a->ntiles = s->ntiles;
+    a->numz = g->numz;
+    a->numw = s->numw1;
+    a->rh0 = 2 * fund_rlo(g->rlo);
+    a->rh_off = g->inmem ? 0 : s->rh_off;
+    a->bstart = g->inmem ? NULL : s->d_bstart;
+    a->corr_uselen = g->corr_uselen;
+    a->nblocks = g->nblocks;
+    a->nstages = g->numharmstages;
+    a->inmem = g->inmem;
+    for (int i = 0; i < g->numharmstages; i++)
+        a->powcut[i] = g->powcut[i];
+    a->nfrac = s->nfrac;
+    a->zmap = s->d_zmap;
+    a->wmap = s->d_wmap;
+    a->row_tab = s->d_rowtab;
+    a->chunk_base = s->d_cbase;
+    a->chunk_lo = s->d_clo;
+    a->nsq = s->d_nsq;
+    a->nsq_hb = s->d_nsq_hb;
+    a->npre = s->npre;
+    a->hits = s->d_hits;
+    a->nhits = s->d_nhits;
+    a->cap = s->cap;
+}
+
 static int search_init(accel_search *s, int device, int nstreams)
 {
     accel_geom *g = &s->g;
@@ -643,7 +676,8 @@ static int search_init(accel_search *s, int device, int nstreams)
         set_err("kernel width %d too large for %d-point segments", 4 * s->hw, s->L);
         return -1;
     }
-    s->uselen = (s->L - 4 * s->hw) & ~1;
+    s->hw += s->hw & 1;   /* segments of whole groups of half-bins (agpu.h) */
+    s->uselen = s->L - 4 * s->hw;
     if (block_starts(s))
         return -1;
     s->hb_end = 2 * fund_rlo(g->rlo) + (long long) g->nblocks * g->corr_uselen;
@@ -700,6 +734,15 @@ static int search_init(accel_search *s, int device, int nstreams)
              agpu_h2d(s->d_cbase, cbase, sizeof(long long) * AGPU_HS_CT * (size_t) nchunks,
                       s->stream) ||
              agpu_h2d(s->d_clo, clo, sizeof(int) * AGPU_HS_CT * (size_t) nchunks, s->stream);
+    s->bounds = !s->d_bstart && !(s->rh_off && !g->inmem) &&
+                agpu_harmbound_pays(g->numharmstages, g->powcut, g->corr_uselen, g->numz,
+                                    s->numw1, ncell, s->nfrac, zmap);
+    if (s->bounds && rc == 0) {
+        agpu_harmsum_args a;
+        fill_harmsum_args(s, &a);
+        const long long nc = agpu_harmbound_chunks(&a);
+        rc = agpu_malloc((void **) &s->d_nb, sizeof(float) * 32 * (size_t) (nc > 0 ? nc : 1));
+    }
     free(rowtab);
     free(cbase);
     free(clo);
@@ -749,6 +792,7 @@ void accel_search_destroy(accel_search *s)
     agpu_free(s->d_norm);
     agpu_free(s->d_nsq);
     agpu_free(s->d_nsq_hb);
+    agpu_free(s->d_nb);
     agpu_free(s->d_zmap);
     agpu_free(s->d_wmap);
     agpu_free(s->d_rowtab);
@@ -807,35 +851,9 @@ int accel_search_set_device_spectrum(accel_search *s, const void *d_fft)
     return 0;
 }
 
-static void fill_harmsum_args(const accel_search *s, agpu_harmsum_args *a)
+static int harmsum(accel_search *s, const agpu_harmsum_args *a)
 {
-    const accel_geom *g = &s->g;
-    memset(a, 0, sizeof(*a));
-    a->plane = s->d_plane;
-    a->ntiles = s->ntiles;
-    a->numz = g->numz;
-    a->numw = s->numw1;
-    a->rh0 = 2 * fund_rlo(g->rlo);
-    a->rh_off = g->inmem ? 0 : s->rh_off;
-    a->bstart = g->inmem ? NULL : s->d_bstart;
-    a->corr_uselen = g->corr_uselen;
-    a->nblocks = g->nblocks;
-    a->nstages = g->numharmstages;
-    a->inmem = g->inmem;
-    for (int i = 0; i < g->numharmstages; i++)
-        a->powcut[i] = g->powcut[i];
-    a->nfrac = s->nfrac;
-    a->zmap = s->d_zmap;
-    a->wmap = s->d_wmap;
-    a->row_tab = s->d_rowtab;
-    a->chunk_base = s->d_cbase;
-    a->chunk_lo = s->d_clo;
-    a->nsq = s->d_nsq;
-    a->nsq_hb = s->d_nsq_hb;
-    a->npre = s->npre;
-    a->hits = s->d_hits;
-    a->nhits = s->d_nhits;
-    a->cap = s->cap;
+    return s->bounds ? agpu_harmbound(a, s->d_nb, s->stream) : agpu_harmsum(a, 0, -1, s->stream);
 }
 
 int accel_search_launch(accel_search *s)
@@ -861,17 +879,20 @@ int accel_search_launch(accel_search *s)
     if (g->inmem)
         GPU(agpu_inmem_nsq_table(s->d_nsq, s->npre, g->nblocks, 2 * fund_rlo(g->rlo),
                                  g->corr_uselen, s->hb_end, s->d_nsq_hb, s->stream2));
+    fill_harmsum_args(s, &a);
+    if (s->bounds)
+        GPU(agpu_bound_norms(&a, s->hb_end, s->d_nb, s->stream2));
     GPU(agpu_event_record(s->ev_norms, s->stream2));
     GPU(agpu_event_record(s->ev[1], s->stream));
     GPU(agpu_correlate(s->d_spec, g->numbins, g->lobin, s->d_T, s->nt, s->L, s->hw, s->uselen,
-                       s->hb_end, s->d_plane, s->ntiles, s->groups, 0, -1, s->stream));
+                       s->hb_end, s->d_plane, s->ntiles, s->groups, 0, -1, s->bounds,
+                       s->stream));
     GPU(agpu_event_record(s->ev[2], s->stream));
     /* the tile halos are written by the correlation itself */
     GPU(agpu_event_record(s->ev[3], s->stream));
     if (two)
         GPU(agpu_stream_wait_event(s->stream, s->ev_norms));
-    fill_harmsum_args(s, &a);
-    GPU(agpu_harmsum(&a, 0, -1, s->stream));
+    GPU(harmsum(s, &a));
     GPU(agpu_event_record(s->ev[4], s->stream));
     s->hms[0] = now_ms() - t0;
     return 0;
@@ -1146,7 +1167,7 @@ int accel_search_collect(accel_search *s)
         agpu_harmsum_args a;
         GPU(agpu_memset(s->d_nhits, 0, sizeof(unsigned), s->stream));
         fill_harmsum_args(s, &a);
-        GPU(agpu_harmsum(&a, 0, -1, s->stream));
+        GPU(harmsum(s, &a));
         GPU(agpu_d2h(&nh, s->d_nhits, sizeof(unsigned), s->stream));
         if (nh > s->cap) {
             set_err("hit buffer overflow after regrowth (%u > %u)", nh, s->cap);
@@ -1323,7 +1344,7 @@ int accel_search_tune(accel_search *s, int ncand, int *groups, float *ms, int *b
             GPU(agpu_event_record(s->ev[1], s->stream));
             GPU(agpu_correlate(s->d_spec, g->numbins, g->lobin, s->d_T, s->nt, s->L, s->hw,
                                s->uselen, s->hb_end, s->d_plane, s->ntiles, cand[i], 0, -1,
-                               s->stream));
+                               s->bounds, s->stream));
             GPU(agpu_event_record(s->ev[2], s->stream));
             GPU(agpu_stream_sync(s->stream));
             GPU(agpu_event_elapsed(&t, s->ev[1], s->ev[2]));
@@ -1694,7 +1715,8 @@ int accel_search_plane_only(accel_search *s)
 {
     const accel_geom *g = &s->g;
     GPU(agpu_correlate(s->d_spec, g->numbins, g->lobin, s->d_T, s->nt, s->L, s->hw, s->uselen,
-                       s->hb_end, s->d_plane, s->ntiles, s->groups, 0, -1, s->stream));
+                       s->hb_end, s->d_plane, s->ntiles, s->groups, 0, -1, s->bounds,
+                       s->stream));
     GPU(agpu_stream_sync(s->stream));
     return 0;
 }

@@ -49,6 +49,14 @@ typedef struct {
     (((size_t) ((hb) >> AGPU_TILE_LOG2) * (size_t) (nrows) + (size_t) (row)) *         \
          (size_t) AGPU_ROWLEN + (size_t) ((hb) & (AGPU_TILE - 1)))
 
+/* In place of the halo a search by bounds (agpu_harmbound) keeps, behind
+ * each tile-row, the largest power of every AGPU_GROUP half-bins as the high
+ * 16 bits of its FP32 value, rounded up: AGPU_TILE / AGPU_GROUP of the tile,
+ * then the first AGPU_BHALO of the next tile. */
+#define AGPU_GROUP_LOG2 2
+#define AGPU_GROUP (1 << AGPU_GROUP_LOG2)
+#define AGPU_BHALO (2 * AGPU_HALO - AGPU_TILE / AGPU_GROUP)
+
 #define AGPU_MAX_FRACS 32
 #define AGPU_MAX_STAGES 6
 
@@ -206,17 +214,26 @@ int agpu_sf_locpow_plane_tab(const void *d_wdata, int numdata, int binoffset, in
 
 /* Fused overlap-save correlation: raw |corr|^2 plane rows for templates
  * [0, nt) (row = template), half-bins [0, hb_end), segment length L = 4096,
- * written in the tiled layout above, halos included.  Only segments [seg_lo, seg_hi)
+ * written in the tiled layout above, with the halos or (bounds) the group
+ * bounds behind each tile-row; bounds need hw even.  Only segments [seg_lo, seg_hi)
  * (segment s: half-bins [s uselen, (s+1) uselen); seg_hi -1: to the end). */
 int agpu_correlate(const void *d_spec, long long numbins, long long lobin_file,
                    const void *d_T, int nt, int L, int hw, int uselen, long long hb_end,
                    float *d_plane, long long ntiles, int groups, long long seg_lo,
-                   long long seg_hi, void *stream);
+                   long long seg_hi, int bounds, void *stream);
 
 /* Harmonic sums of fundamental chunks [c_lo, c_hi) (-1: to the end); chunk
  * c covers the 1024 half-bins from agpu_harmsum_chunk_hb(a, c). */
 int agpu_harmsum(const agpu_harmsum_args *a, long long c_lo, long long c_hi, void *stream);
 long long agpu_harmsum_nchunks(const agpu_harmsum_args *a);
+/* The same hits from a plane with group bounds: whether it pays for these
+ * thresholds, the chunks of its norm table d_nb ([chunks][32] floats), the
+ * table (after the norms), the search. */
+int agpu_harmbound_pays(int nstages, const float *powcut, int corr_uselen, int numz, int numw,
+                        long long numhb, int nfrac, const int *zmap);
+long long agpu_harmbound_chunks(const agpu_harmsum_args *a);
+int agpu_bound_norms(const agpu_harmsum_args *a, long long hb_end, float *d_nb, void *stream);
+int agpu_harmbound(const agpu_harmsum_args *a, const float *d_nb, void *stream);
 long long agpu_harmsum_chunk_hb(const agpu_harmsum_args *a, long long c);
 
 /* In-memory path: per-half-bin norm^2 of the block that last wrote it. */

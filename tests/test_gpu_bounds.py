@@ -1,0 +1,110 @@
+"""The harmonic sum by bounds (k_harmbound) against the sums themselves:
+every hit recomputed in numpy from the search's raw plane and norms, term by
+term in FP32 in the order of the fractions, so set and powers must be equal.
+The shapes are those at which it can go wrong: 1 to 5 stages, both index
+rules, row blocks below, at and above 64 rows, jerk rows, ragged lengths, a
+first half-bin off every chunk edge, strong signals, bins without power,
+infinities and NaN."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+A = pytest.importorskip("presto_amd.accel")
+
+# agpu_harmbound_pays: thresholds high enough for their harmonics, 16 rows, 2^23 cells
+def _by_bounds(g):
+    numw = max(g.numw, 1)
+    cells = g.numz * numw * g.nblocks * g.corr_uselen
+    H = 2.0 ** np.arange(g.numharmstages)
+    cut = np.array(list(g.powcut))[:g.numharmstages]
+    return g.numz >= 16 and cells >= 1 << 23 and bool((cut >= 2.13 * H + 3.1 * np.sqrt(H)).all())
+
+
+def _nearest(x):
+    return np.where(x < 0, np.ceil(x - 0.5), np.floor(x + 0.5)).astype(int)
+
+
+def _expected(s):
+    g = s.geom
+    numw = max(g.numw, 1)
+    ncell = g.nblocks * g.corr_uselen
+    rh0 = 2 * int(np.floor(np.rint(2 * g.rlo) / 2))
+    plane = np.stack([np.stack([s.plane_row(w, z, 0, rh0 + ncell) for z in range(g.numz)])
+                      for w in range(numw)])
+    norm = s.norms()
+    nsq = (norm * norm).astype(np.float32)
+    rh = rh0 + np.arange(ncell)
+    block = np.arange(ncell) // g.corr_uselen
+    if g.inmem:
+        npre = len(norm) - g.nblocks
+        hb = np.arange(rh0 + ncell)
+        owner = np.where(hb >= rh0, npre + (hb - rh0) // g.corr_uselen, (hb - 16) // g.corr_uselen)
+        nsq_hb = np.where((hb < 16) & (hb < rh0), np.float32(0), nsq[owner.clip(0)])
+    nfr = 1 << (g.numharmstages - 1)
+    zs = g.zlo + 2.0 * np.arange(g.numz)
+    ws = g.wlo + 20.0 * np.arange(numw)
+    hits = []
+    acc, f = None, 0
+    for st in range(g.numharmstages):
+        H = 1 << st
+        for k in range(1, H + (st == 0), 2):
+            q = rh * k
+            rs = (q + H // 2) // H if g.inmem else np.rint(q / H).astype(np.int64)
+            zi = ((2 * _nearest(0.5 * zs * k / H) + g.zhi) / 2).astype(int)
+            wi = ((20 * _nearest(0.05 * ws * k / H) + g.whi) / 20).astype(int) if g.numw else [0]
+            n = nsq_hb[rs] if g.inmem else nsq.reshape(g.nblocks, nfr)[block, f]
+            with np.errstate(all="ignore"):
+                term = plane[np.ix_(wi, zi)][:, :, rs] * n
+                acc = term if acc is None else acc + term
+            f += 1
+        with np.errstate(all="ignore"):
+            for w, z, c in np.argwhere(acc > np.float32(g.powcut[st])):
+                hits.append((int(c) // g.corr_uselen, st, int(w), int(z), int(c) % g.corr_uselen,
+                             acc[w, z, c]))
+    return sorted(hits, key=lambda h: h[:5])
+
+
+def _spectrum(nbins, seed, signals=(), odd=None):
+    rng = np.random.Generator(np.random.PCG64(seed))
+    X = (rng.standard_normal(nbins) + 1j * rng.standard_normal(nbins)) / np.sqrt(2.0)
+    for r, amp in signals:
+        X[r] += amp
+    X = X.astype(np.complex64)
+    X[0] = 1 + 1j
+    if odd == "zeros":
+        X[nbins // 2:nbins // 2 + 6000] = 0
+    if odd == "inf":
+        X[nbins // 2] = np.inf
+        X[nbins // 3] = complex(np.nan, 1.0)
+    return X
+
+
+@pytest.mark.parametrize("nbins,zmax,wmax,numharm,inmem,rlo,odd", [
+    (150000, 30, None, 1, False, 100, None),
+    (150000, 30, None, 2, True, 101, None),
+    (100001, 63, None, 4, False, 333, None),          # 64 rows, one block
+    (100001, 64, None, 4, True, 333, None),           # 65 rows, two
+    (1 << 17, 50, None, 8, True, 21, None),
+    (1 << 17, 50, None, 8, False, 22, "zeros"),
+    (1 << 17, 50, None, 8, True, 23, "inf"),
+    (1 << 17, 50, None, 8, False, 23, "inf"),
+    (1 << 18, 100, None, 16, False, 77, None),
+    (1 << 18, 100, None, 16, True, 1, None),
+    (60000, 30, 40, 8, False, 50, None),              # 31 x 5 rows
+])
+def test_hits_equal_the_sums(nbins, zmax, wmax, numharm, inmem, rlo, odd):
+    sig = [(nbins // 7, 9.0), (2 * (nbins // 7), 8.0), (3 * (nbins // 7), 7.0),
+           (nbins // 5 + 3, 200.0), (rlo + 5, 12.0)]
+    p = A.make_params(nbins, 2 * nbins, 1e-3, zmax=zmax, numharm=numharm, sigma=2.5, wmax=wmax,
+                      rlo=rlo, rhi=nbins - 1, inmem=inmem, force_standard=not inmem,
+                      dat_input=False)
+    with A.Search(p) as s:
+        assert _by_bounds(s.geom) and bool(s.geom.inmem) == inmem
+        s.set_spectrum(_spectrum(nbins, 11 + numharm, sig, odd))
+        s.run()
+        got = [(int(h["block"]), int(h["stage"]), int(h["wi"]), int(h["zi"]), int(h["ii"]),
+                h["pow"]) for h in s.hits()]
+        want = _expected(s)
+    assert len(want) > 20
+    assert [h[:5] for h in got] == [h[:5] for h in want]
+    np.testing.assert_array_equal(np.array([h[5] for h in got]), np.array([h[5] for h in want]))
