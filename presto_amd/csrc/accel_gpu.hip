@@ -1450,26 +1450,29 @@ static_assert(hb_dw(15, 4) <= 32 && 2 * (AGPU_TILE / AGPU_GROUP + AGPU_BHALO) ==
  * dword t % lpr of row t / lpr (and 256 / lpr rows on). */
 template <int K, int S>
 __device__ __forceinline__ void hb_load(const agpu_harmsum_args &a, unsigned *v, int g0,
-                                        long long tile_stride, int wi, int z0, int z1)
+                                        long long tile_stride, const unsigned *rt0,
+                                        const unsigned *rt1)
 {
     constexpr int LPR = hb_lpr(K, S), RPP = 256 / LPR, F = S ? (1 << S >> 1) + (K - 1) / 2 : 0;
     const int J = g0 * K >> S;   /* exact: g0 is a multiple of 64 */
-    const int zf = S ? a.zmap[(F - 1) * a.numz + z0] : z0;
-    const int nr = (S ? a.zmap[(F - 1) * a.numz + z1 - 1] : z1 - 1) - zf + 1;
-    const int wf = S ? a.wmap[(F - 1) * a.numw + wi] : wi;
+    const unsigned r0 = rt0[S ? HS_RT_SUB + F - 1 : HS_RT_ROW];
+    const unsigned r1 = rt1[S ? HS_RT_SUB + F - 1 : HS_RT_ROW];
     const char *base = (const char *) (a.plane +
                                        (long long) (J >> (AGPU_TILE_LOG2 - AGPU_GROUP_LOG2)) *
-                                           tile_stride +
-                                       ((long long) wf * a.numz + zf) * AGPU_ROWLEN + AGPU_TILE) +
+                                           tile_stride + r0 + AGPU_TILE) +
                        2 * (J & (AGPU_TILE / AGPU_GROUP - 1));
+    /* through a descriptor that ends with the last row: a load past it (or
+     * of a dword past the row's) is out of range and returns 0 */
+    const unsigned bytes = 4u * (r1 - r0 + hb_dw(K, S));
+    const __amdgpu_buffer_rsrc_t rs =
+        __builtin_amdgcn_make_buffer_rsrc((void *) base, 0, (int) bytes, 0x00027000);
     const int dw = threadIdx.x % LPR, row = threadIdx.x / LPR;
-    const unsigned off = (unsigned) (row * 4 * AGPU_ROWLEN + 4 * dw);
+    const unsigned off = S == 0 || dw < hb_dw(K, S)
+                             ? 4u * (unsigned) (row * AGPU_ROWLEN + dw) : 0x80000000u;
 #pragma unroll
-    for (int u = 0; u < hb_loads(K, S); u++) {
-        v[u] = 0;
-        if (row + u * RPP < nr && (S == 0 || dw < hb_dw(K, S)))
-            v[u] = *(const unsigned *) (base + (off + (unsigned) (u * RPP * 4 * AGPU_ROWLEN)));
-    }
+    for (int u = 0; u < hb_loads(K, S); u++)
+        v[u] = __builtin_amdgcn_raw_buffer_load_b32(rs, (int) (off + 4u * u * RPP * AGPU_ROWLEN),
+                                                    0, 0);
 }
 
 template <int K, int S>
@@ -1509,6 +1512,15 @@ __device__ __forceinline__ void hb_add(float *acc, const unsigned *p, float nn)
     }
 }
 
+/* The sub-harmonic z row of row z (from the middle row) for fraction
+ * k / 2^s, from the middle row: k z / 2^s rounded half away from zero, as
+ * calc_required_z rounds it (src/accel_utils.c:65). */
+__host__ __device__ __forceinline__ int hb_zmap(int z, int k, int s)
+{
+    const int m = z * k, h = 1 << s >> 1;
+    return m < 0 ? -((h - m) >> s) : (h + m) >> s;
+}
+
 /* any of the 16 sums above the threshold, or NaN */
 __device__ __forceinline__ bool hb_over(const float *acc, float cut)
 {
@@ -1522,11 +1534,12 @@ __device__ __forceinline__ bool hb_over(const float *acc, float cut)
 /* stage by stage, the fractions of a stage in order */
 template <int K, int S>
 __device__ __forceinline__ void hb_load_stage(const agpu_harmsum_args &a, unsigned *v, int g0,
-                                              long long tile_stride, int wi, int z0, int z1)
+                                              long long tile_stride, const unsigned *rt0,
+                                              const unsigned *rt1)
 {
-    hb_load<K, S>(a, v, g0, tile_stride, wi, z0, z1);
+    hb_load<K, S>(a, v, g0, tile_stride, rt0, rt1);
     if constexpr (K + 2 < (1 << S))
-        hb_load_stage<K + 2, S>(a, v + hb_loads(K, S), g0, tile_stride, wi, z0, z1);
+        hb_load_stage<K + 2, S>(a, v + hb_loads(K, S), g0, tile_stride, rt0, rt1);
 }
 template <int K, int S>
 __device__ __forceinline__ void hb_store_stage(unsigned *lds, const unsigned *v)
@@ -1536,15 +1549,14 @@ __device__ __forceinline__ void hb_store_stage(unsigned *lds, const unsigned *v)
         hb_store_stage<K + 2, S>(lds + hb_dw(K, S) * hb_nr(K, S), v + hb_loads(K, S));
 }
 template <int K, int S, bool ODD>
-__device__ __forceinline__ void hb_add_stage(const agpu_harmsum_args &a, float *acc,
-                                             const unsigned *lds, const float *np, int z0, int z,
-                                             int wv)
+__device__ __forceinline__ void hb_add_stage(float *acc, const unsigned *lds, const float *np,
+                                             int z0, int z, int wv)
 {
     constexpr int F = (1 << S >> 1) + (K - 1) / 2;
-    const int zs = a.zmap[(F - 1) * a.numz + z] - a.zmap[(F - 1) * a.numz + z0];
+    const int zs = hb_zmap(z, K, S) - hb_zmap(z0, K, S);
     hb_add<K, S, ODD>(acc, lds + zs * hb_dw(K, S) + (wv * (16 * K >> S)) / 2, np[F]);
     if constexpr (K + 2 < (1 << S))
-        hb_add_stage<K + 2, S, ODD>(a, acc, lds + hb_dw(K, S) * hb_nr(K, S), np, z0, z, wv);
+        hb_add_stage<K + 2, S, ODD>(acc, lds + hb_dw(K, S) * hb_nr(K, S), np, z0, z, wv);
 }
 
 /* The harmonic sum and threshold by bounds.  A workgroup takes 256
@@ -1589,16 +1601,19 @@ __global__ __launch_bounds__(256) void k_harmbound(agpu_harmsum_args a, const fl
     const int hb = ((int) a.rh0 / HB_CHUNK + c) * HB_CHUNK, g0 = hb / AGPU_GROUP;
     const long long tile_stride = (long long) a.numz * a.numw * AGPU_ROWLEN;
     const float *np = nb + (size_t) c * 32;
+    /* the first and the last row's tables: where a fraction's rows begin and end */
+    const unsigned *rt0 = a.row_tab + (size_t) (wi * a.numz + z0) * HS_RT;
+    const unsigned *rt1 = a.row_tab + (size_t) (wi * a.numz + z1 - 1) * HS_RT;
     constexpr int LAST = NSTAGES < 4 ? NSTAGES - 1 : 3;
     {
         unsigned v[hb_nloads(0, LAST)];
-        hb_load<1, 0>(a, v, g0, tile_stride, wi, z0, z1);
+        hb_load<1, 0>(a, v, g0, tile_stride, rt0, rt1);
         if constexpr (NSTAGES > 1)
-            hb_load_stage<1, 1>(a, v + hb_nloads(0, 0), g0, tile_stride, wi, z0, z1);
+            hb_load_stage<1, 1>(a, v + hb_nloads(0, 0), g0, tile_stride, rt0, rt1);
         if constexpr (NSTAGES > 2)
-            hb_load_stage<1, 2>(a, v + hb_nloads(0, 1), g0, tile_stride, wi, z0, z1);
+            hb_load_stage<1, 2>(a, v + hb_nloads(0, 1), g0, tile_stride, rt0, rt1);
         if constexpr (NSTAGES > 3)
-            hb_load_stage<1, 3>(a, v + hb_nloads(0, 2), g0, tile_stride, wi, z0, z1);
+            hb_load_stage<1, 3>(a, v + hb_nloads(0, 2), g0, tile_stride, rt0, rt1);
         hb_store<1, 0>(lds, v);
         if constexpr (NSTAGES > 1)
             hb_store_stage<1, 1>(lds + hb_base(0, 1, 1), v + hb_nloads(0, 0));
@@ -1609,22 +1624,22 @@ __global__ __launch_bounds__(256) void k_harmbound(agpu_harmsum_args a, const fl
     }
     unsigned v4[NSTAGES > 4 ? hb_nloads(4, 4) : 1];
     if constexpr (NSTAGES > 4)   /* in flight while the stages before are summed */
-        hb_load_stage<1, 4>(a, v4, g0, tile_stride, wi, z0, z1);
+        hb_load_stage<1, 4>(a, v4, g0, tile_stride, rt0, rt1);
     __syncthreads();
-    const int z = min(z0 + lane, z1 - 1);
+    const int z = min(z0 + lane, z1 - 1), mid = (a.numz - 1) / 2;
     float acc[16];
     hb_add<1, 0, false>(acc, lds + (z - z0) * hb_dw(1, 0) + wv * 8, np[0]);
     bool over = hb_over(acc, a.powcut[0]);
     if constexpr (NSTAGES > 1) {
-        hb_add_stage<1, 1, false>(a, acc, lds + hb_base(0, 1, 1), np, z0, z, wv);
+        hb_add_stage<1, 1, false>(acc, lds + hb_base(0, 1, 1), np, z0 - mid, z - mid, wv);
         over |= hb_over(acc, a.powcut[1]);
     }
     if constexpr (NSTAGES > 2) {
-        hb_add_stage<1, 2, false>(a, acc, lds + hb_base(0, 1, 2), np, z0, z, wv);
+        hb_add_stage<1, 2, false>(acc, lds + hb_base(0, 1, 2), np, z0 - mid, z - mid, wv);
         over |= hb_over(acc, a.powcut[2]);
     }
     if constexpr (NSTAGES > 3) {
-        hb_add_stage<1, 3, false>(a, acc, lds + hb_base(0, 1, 3), np, z0, z, wv);
+        hb_add_stage<1, 3, false>(acc, lds + hb_base(0, 1, 3), np, z0 - mid, z - mid, wv);
         over |= hb_over(acc, a.powcut[3]);
     }
     if constexpr (NSTAGES > 4) {
@@ -1633,9 +1648,9 @@ __global__ __launch_bounds__(256) void k_harmbound(agpu_harmsum_args a, const fl
         __syncthreads();
         /* k groups per wave: an odd wave starts on an odd group */
         if (wv & 1)
-            hb_add_stage<1, 4, true>(a, acc, lds, np, z0, z, wv);
+            hb_add_stage<1, 4, true>(acc, lds, np, z0 - mid, z - mid, wv);
         else
-            hb_add_stage<1, 4, false>(a, acc, lds, np, z0, z, wv);
+            hb_add_stage<1, 4, false>(acc, lds, np, z0 - mid, z - mid, wv);
         over |= hb_over(acc, a.powcut[4]);
     }
     const unsigned long long todo = __ballot(over && z0 + lane < z1);
@@ -2240,8 +2255,8 @@ int agpu_harmbound_pays(int nstages, const float *powcut, int corr_uselen, int n
         for (int z0 = 0; z0 < numz; z0 += zrows) {
             const int z1 = z0 + zrows < numz ? z0 + zrows : numz;
             const int *m = zmap + (size_t) (f - 1) * numz;
-            for (int z = z0 + 1; z < z1; z++)
-                if (m[z] < m[z - 1])
+            for (int z = z0; z < z1; z++)
+                if (m[z] != hb_zmap(z - (numz - 1) / 2, k, s) + (numz - 1) / 2)
                     return 0;
             if (m[z1 - 1] - m[z0] + 1 > hb_nr(k, s))
                 return 0;
@@ -2292,8 +2307,8 @@ int agpu_harmbound(const agpu_harmsum_args *a, const float *d_nb, void *stream)
     if ((rh_end + HS_CHUNK) * (long long) ((1 << (a->nstages - 1)) - 1) > 0x7fffffffLL)
         return fail("agpu_harmbound: spectrum too long for 32-bit sub-harmonic indices "
                     "(half-bins x highest harmonic must stay below 2^31)");
-    if (!a->row_tab || (a->nfrac && (!a->zmap || !a->wmap)))
-        return fail("agpu_harmbound: row tables missing");
+    if (!a->row_tab)
+        return fail("agpu_harmbound: row table missing");
     if ((long long) a->numz * a->numw * AGPU_ROWLEN > 0x3fffffffLL)
         return fail("agpu_harmbound: too many rows for 32-bit row offsets");
     const int zrows = hb_zrows(a->numz), zblocks = (a->numz + zrows - 1) / zrows;
