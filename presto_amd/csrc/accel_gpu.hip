@@ -50,6 +50,9 @@ static int fail(const char *msg)
 }
 
 #include "dev_fresnel.h"
+#define ACCEL_SIGMA_FN __device__ static
+#define ACCEL_SIGMA_TOL 1e-15
+#include "accel_sigma.h"
 
 #define CORR_N 4096   /* half-bins per correlation segment */
 
@@ -957,7 +960,7 @@ __device__ __forceinline__ void emit_hit(const agpu_harmsum_args &a, int b, int 
         h.zi = zi;
         h.ii = ii;
         h.pow = p;
-        a.hits[idx] = h;
+        a.hits[idx].h = h;
     }
 }
 
@@ -1288,6 +1291,20 @@ __global__ __launch_bounds__(HS_TPB) void k_harmsum(agpu_harmsum_args a, int c_l
     }
 #undef HS_STAGE
 #undef HS_EMIT
+}
+
+/* Sigma of every hit (src/accel_utils.c:1434-1437), one thread per hit:
+ * FP64 Newton steps on log(erfc), ~1 us each on a host core, here all at
+ * once behind the harmonic sum (~12 us for any count up to some thousands).
+ * A fixed grid strides over the count that the sum left on the device. */
+__global__ __launch_bounds__(64) void k_hit_sigmas(agpu_hitrec *hits, const unsigned *nhits,
+                                                   unsigned cap, agpu_numindep ni)
+{
+    const unsigned n = min(*nhits, cap);
+    for (unsigned i = blockIdx.x * 64 + threadIdx.x; i < n; i += gridDim.x * 64) {
+        const agpu_hit h = hits[i].h;
+        hits[i].sigma = (float) sigma_of_power(h.pow, 1 << h.stage, ni.n[h.stage]);
+    }
 }
 
 /* ---- the harmonic sum over bounds ---- */
@@ -2335,6 +2352,15 @@ int agpu_harmbound(const agpu_harmsum_args *a, const float *d_nb, void *stream)
         HB_CASE(5)
     }
 #undef HB_CASE
+    AGPU_CHECK(hipGetLastError());
+    return 0;
+}
+
+int agpu_hit_sigmas(agpu_hitrec *d_hits, const unsigned *d_nhits, unsigned cap,
+                    const agpu_numindep *ni, void *stream)
+{
+    hipLaunchKernelGGL(k_hit_sigmas, dim3(1024), dim3(64), 0, (hipStream_t) stream, d_hits,
+                       d_nhits, cap, *ni);
     AGPU_CHECK(hipGetLastError());
     return 0;
 }

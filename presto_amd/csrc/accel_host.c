@@ -13,7 +13,7 @@
  *              (w,z) row (AGPU_PLANE_IDX)             un-normalised |corr|^2
  *   windows    {lobin, numdata}[nwin] -> norm (FP64), nsq = norm^2 (FP32)
  *   zmap/wmap  int[nfrac][numz] / int[nfrac][numw']  sub-harmonic rows
- *   hits       accel_hit[cap] + counter
+ *   hits       counter + agpu_hitrec[cap] (hit, sigma)
  * Correlation is linear, so the reference's normalised plane of any block
  * and any harmonic fraction is norm^2 times the raw plane at the same
  * (r, z, w); the harmonic-sum kernel applies the norm of the window that
@@ -34,7 +34,7 @@
 
 #define MAXRAMUSE 2000000000LL
 #define CORR_L 4096
-#define HIT_CAP0 (1u << 20)
+#define HIT_CAP0 (3u << 18)   /* 24 MiB of records */
 
 static __thread char g_err[1024];   /* per host thread */
 
@@ -328,8 +328,8 @@ struct accel_search {
     unsigned *d_rowtab;   /* harmonic-sum address tables (agpu.h) */
     long long *d_cbase;
     int *d_clo;
-    agpu_hit *d_hits;
-    unsigned *d_nhits;
+    agpu_hitrec *d_hits;   /* one record ahead of the hits: the hit count */
+    unsigned *d_nhits;     /* (d_hits and d_nhits: one allocation, see alloc_hits) */
     unsigned cap;
     /* block start r, accumulated as src/accelsearch.c:189-224 does; a
      * fractional -rlo makes the sub-harmonic lookups depend on it */
@@ -339,6 +339,7 @@ struct accel_search {
     FILE *workfile;       /* .txtcand of an .fft input, or NULL */
     /* results */
     accel_hit *hits;
+    float *sigs;          /* the hits' sigmas */
     long long nhits;
     cnode *cands;
     int ncands;
@@ -656,6 +657,21 @@ static void fill_harmsum_args(const accel_search *s, agpu_harmsum_args *a)
     a->cap = s->cap;
 }
 
+/* The hit buffer: the count in its first record, then the hits, so that one
+ * copy brings back the count and the first hits. */
+static int alloc_hits(accel_search *s, unsigned cap)
+{
+    void *d = NULL;
+    s->d_hits = NULL;
+    s->d_nhits = NULL;
+    s->cap = 0;
+    GPU(agpu_malloc(&d, sizeof(agpu_hitrec) * ((size_t) cap + 1)));
+    s->d_nhits = (unsigned *) d;
+    s->d_hits = (agpu_hitrec *) d + 1;
+    s->cap = cap;
+    return 0;
+}
+
 static int search_init(accel_search *s, int device, int nstreams)
 {
     accel_geom *g = &s->g;
@@ -704,9 +720,8 @@ static int search_init(accel_search *s, int device, int nstreams)
     int nf = s->nfrac > 0 ? s->nfrac : 1;
     GPU(agpu_malloc((void **) &s->d_zmap, sizeof(int) * (size_t) nf * g->numz));
     GPU(agpu_malloc((void **) &s->d_wmap, sizeof(int) * (size_t) nf * s->numw1));
-    s->cap = HIT_CAP0;
-    GPU(agpu_malloc((void **) &s->d_hits, sizeof(agpu_hit) * s->cap));
-    GPU(agpu_malloc((void **) &s->d_nhits, sizeof(unsigned)));
+    if (alloc_hits(s, HIT_CAP0))
+        return -1;
     GPU(agpu_h2d(s->d_win, win, sizeof(agpu_window) * (size_t) (s->nwin > 0 ? s->nwin : 1), s->stream));
     if (g->nph > 0.0 && photon_norms(s))
         return -1;
@@ -798,8 +813,8 @@ void accel_search_destroy(accel_search *s)
     agpu_free(s->d_rowtab);
     agpu_free(s->d_cbase);
     agpu_free(s->d_clo);
-    agpu_free(s->d_hits);
     agpu_free(s->d_nhits);
+    free(s->sigs);
     agpu_free(s->d_bstart);
     free(s->bstart);
     if (s->workfile)
@@ -856,6 +871,15 @@ static int harmsum(accel_search *s, const agpu_harmsum_args *a)
     return s->bounds ? agpu_harmbound(a, s->d_nb, s->stream) : agpu_harmsum(a, 0, -1, s->stream);
 }
 
+static int hit_sigmas(accel_search *s)
+{
+    agpu_numindep ni;
+    memset(&ni, 0, sizeof(ni));
+    for (int i = 0; i < s->g.numharmstages; i++)
+        ni.n[i] = (double) s->g.numindep[i];
+    return agpu_hit_sigmas(s->d_hits, s->d_nhits, s->cap, &ni, s->stream);
+}
+
 int accel_search_launch(accel_search *s)
 {
     const accel_geom *g = &s->g;
@@ -894,13 +918,14 @@ int accel_search_launch(accel_search *s)
         GPU(agpu_stream_wait_event(s->stream, s->ev_norms));
     GPU(harmsum(s, &a));
     GPU(agpu_event_record(s->ev[4], s->stream));
+    GPU(hit_sigmas(s));
     s->hms[0] = now_ms() - t0;
     return 0;
 }
 
 static int cmp_hit(const void *pa, const void *pb)
 {
-    const accel_hit *a = (const accel_hit *) pa, *b = (const accel_hit *) pb;
+    const agpu_hit *a = &((const agpu_hitrec *) pa)->h, *b = &((const agpu_hitrec *) pb)->h;
     if (a->block != b->block) return a->block < b->block ? -1 : 1;
     if (a->stage != b->stage) return a->stage < b->stage ? -1 : 1;
     if (a->wi != b->wi) return a->wi < b->wi ? -1 : 1;
@@ -926,16 +951,16 @@ static int bits_for(unsigned v)
  * into one 64-bit key (widths from the largest value of each field) and
  * sorted by an LSD radix sort of 11-bit digits.  Falls back to qsort if a
  * field is negative or the key would not fit. */
-static int sort_hits(accel_hit *h, long long n)
+static int sort_hits(agpu_hitrec *h, long long n)
 {
     if (n < 2)
         return 0;
     unsigned mx[5] = {0, 0, 0, 0, 0};
     for (long long i = 0; i < n; i++) {
-        const int f[5] = {h[i].block, h[i].stage, h[i].wi, h[i].zi, h[i].ii};
+        const int f[5] = {h[i].h.block, h[i].h.stage, h[i].h.wi, h[i].h.zi, h[i].h.ii};
         for (int k = 0; k < 5; k++) {
             if (f[k] < 0) {
-                qsort(h, (size_t) n, sizeof(accel_hit), cmp_hit);
+                qsort(h, (size_t) n, sizeof(agpu_hitrec), cmp_hit);
                 return 0;
             }
             if ((unsigned) f[k] > mx[k])
@@ -946,12 +971,12 @@ static int sort_hits(accel_hit *h, long long n)
     for (int k = 0; k < 5; k++)
         tot += nb[k] = bits_for(mx[k]);
     if (tot > 64 || n > 0xffffffffLL) {
-        qsort(h, (size_t) n, sizeof(accel_hit), cmp_hit);
+        qsort(h, (size_t) n, sizeof(agpu_hitrec), cmp_hit);
         return 0;
     }
     unsigned long long *key = (unsigned long long *) malloc(sizeof(unsigned long long) * 2 * n);
     unsigned *idx = (unsigned *) malloc(sizeof(unsigned) * 2 * n);
-    accel_hit *tmp = (accel_hit *) malloc(sizeof(accel_hit) * n);
+    agpu_hitrec *tmp = (agpu_hitrec *) malloc(sizeof(agpu_hitrec) * n);
     if (!key || !idx || !tmp) {
         free(key);
         free(idx);
@@ -960,8 +985,8 @@ static int sort_hits(accel_hit *h, long long n)
         return -1;
     }
     for (long long i = 0; i < n; i++) {
-        const unsigned f[5] = {(unsigned) h[i].block, (unsigned) h[i].stage, (unsigned) h[i].wi,
-                               (unsigned) h[i].zi, (unsigned) h[i].ii};
+        const unsigned f[5] = {(unsigned) h[i].h.block, (unsigned) h[i].h.stage,
+                               (unsigned) h[i].h.wi, (unsigned) h[i].h.zi, (unsigned) h[i].h.ii};
         unsigned long long kv = 0;
         for (int k = 0; k < 5; k++)
             kv = (nb[k] ? (kv << nb[k]) : kv) | f[k];
@@ -996,66 +1021,15 @@ static int sort_hits(accel_hit *h, long long n)
     }
     for (long long i = 0; i < n; i++)
         tmp[i] = h[ia[i]];
-    memcpy(h, tmp, sizeof(accel_hit) * n);
+    memcpy(h, tmp, sizeof(agpu_hitrec) * n);
     free(key);
     free(idx);
     free(tmp);
     return 0;
 }
 
-/* Sigma of every hit (src/accel_utils.c:1434-1437), spread over host
- * threads when there are many: each value is a pure function of its hit,
- * so the result does not depend on the split. */
-typedef struct {
-    const accel_hit *h;
-    const accel_geom *g;
-    float *sig;
-    long long lo, hi;
-} sig_job;
-
-static void *sig_worker(void *arg)
-{
-    sig_job *j = (sig_job *) arg;
-    for (long long i = j->lo; i < j->hi; i++) {
-        const accel_hit *h = &j->h[i];
-        j->sig[i] = (float) accel_candidate_sigma(h->pow, 1 << h->stage,
-                                                  (double) j->g->numindep[h->stage]);
-    }
-    return NULL;
-}
-
 #define SIG_MAX_THREADS 16
 #define SIG_PER_THREAD 128   /* ~1 us per sigma: threads pay off above a few hundred hits */
-
-static void hit_sigmas(const accel_hit *h, long long n, const accel_geom *g, float *sig)
-{
-    long np = sysconf(_SC_NPROCESSORS_ONLN);
-    long long nt = n / SIG_PER_THREAD;
-    if (nt > np)
-        nt = np;
-    if (nt > SIG_MAX_THREADS)
-        nt = SIG_MAX_THREADS;
-    sig_job jb[SIG_MAX_THREADS];
-    pthread_t th[SIG_MAX_THREADS];
-    int started[SIG_MAX_THREADS] = {0};
-    if (nt < 2) {
-        sig_job one = {h, g, sig, 0, n};
-        sig_worker(&one);
-        return;
-    }
-    for (int t = 0; t < nt; t++) {
-        jb[t] = (sig_job){h, g, sig, n * t / nt, n * (t + 1) / nt};
-        if (t > 0)
-            started[t] = pthread_create(&th[t], NULL, sig_worker, &jb[t]) == 0;
-    }
-    sig_worker(&jb[0]);
-    for (int t = 1; t < nt; t++) {
-        if (started[t])
-            pthread_join(th[t], NULL);
-        else
-            sig_worker(&jb[t]);
-    }
-}
 
 typedef struct {
     const float *pow;
@@ -1108,14 +1082,7 @@ void accel_sigmas(const float *pow, long long n, int numharm, double numindep, f
 static int replay(accel_search *s)
 {
     const accel_geom *g = &s->g;
-    if (sort_hits(s->hits, s->nhits))
-        return -1;
-    float *sigs = (float *) malloc(sizeof(float) * (s->nhits ? s->nhits : 1));
-    if (!sigs) {
-        set_err("out of host memory for %lld hit sigmas", s->nhits);
-        return -1;
-    }
-    hit_sigmas(s->hits, s->nhits, g, sigs);
+    const float *sigs = s->sigs;
     clear_opt(s);
     free_cands(s->cands);
     s->cands = NULL;
@@ -1133,7 +1100,6 @@ static int replay(accel_search *s)
             fprintf(s->workfile, "%-7.2f  %-7.4f  %-2d  %-14.4f  %-14.9f  %-10.4f %-10.4f\n",
                     h->pow, sig, numharm, rr, rr / g->T, zz, ww);
     }
-    free(sigs);
     int n = 0;
     for (cnode *c = s->cands; c; c = c->next)
         n++;
@@ -1147,47 +1113,86 @@ static int replay(accel_search *s)
     return 0;
 }
 
+#define HIT_FIRST 1023   /* hits that come back with the count */
+
 int accel_search_collect(accel_search *s)
 {
-    unsigned nh = 0;
     double t0 = now_ms();
-    GPU(agpu_d2h(&nh, s->d_nhits, sizeof(unsigned), s->stream));
-    if (nh > s->cap) {
+    agpu_hitrec *rec = (agpu_hitrec *) malloc(sizeof(agpu_hitrec) * (HIT_FIRST + 1));
+    if (!rec) {
+        set_err("out of host memory for the hits");
+        return -1;
+    }
+    unsigned first = s->cap < HIT_FIRST ? s->cap : HIT_FIRST, nh;
+    int rc = agpu_d2h(rec, s->d_nhits, sizeof(agpu_hitrec) * ((size_t) first + 1), s->stream);
+    nh = rc ? 0 : *(const unsigned *) rec;
+    if (!rc && nh > s->cap) {
         /* too many crossings for the buffer: grow it and sum again.  The
          * handle never keeps a freed buffer: on a failed allocation it has
          * no hit buffer (cap 0) and refuses to launch until rebuilt. */
-        GPU(agpu_free(s->d_hits));
-        s->d_hits = NULL;
-        s->cap = 0;
         const unsigned cap = nh + nh / 4 + 1024;
-        void *d_new = NULL;
-        GPU(agpu_malloc(&d_new, sizeof(agpu_hit) * cap));
-        s->d_hits = (agpu_hit *) d_new;
-        s->cap = cap;
         agpu_harmsum_args a;
-        GPU(agpu_memset(s->d_nhits, 0, sizeof(unsigned), s->stream));
+        rc = agpu_free(s->d_nhits);
+        if (alloc_hits(s, cap)) {
+            free(rec);
+            return -1;
+        }
         fill_harmsum_args(s, &a);
-        GPU(harmsum(s, &a));
-        GPU(agpu_d2h(&nh, s->d_nhits, sizeof(unsigned), s->stream));
+        rc = rc || agpu_memset(s->d_nhits, 0, sizeof(unsigned), s->stream) || harmsum(s, &a) ||
+             hit_sigmas(s) ||
+             agpu_d2h(rec, s->d_nhits, sizeof(agpu_hitrec) * (HIT_FIRST + 1), s->stream);
+        nh = rc ? 0 : *(const unsigned *) rec;
+        first = HIT_FIRST;
         if (nh > s->cap) {
             set_err("hit buffer overflow after regrowth (%u > %u)", nh, s->cap);
+            free(rec);
             return -1;
         }
     }
-    GPU(agpu_event_elapsed(&s->ms[0], s->ev[0], s->ev_norms));
+    rc = rc || agpu_event_elapsed(&s->ms[0], s->ev[0], s->ev_norms);
     for (int i = 1; i < 4; i++)
-        GPU(agpu_event_elapsed(&s->ms[i], s->ev[i], s->ev[i + 1]));
-    GPU(agpu_event_elapsed(&s->ms[4], s->ev[0], s->ev[4]));
+        rc = rc || agpu_event_elapsed(&s->ms[i], s->ev[i], s->ev[i + 1]);
+    rc = rc || agpu_event_elapsed(&s->ms[4], s->ev[0], s->ev[4]);
     double t1 = now_ms();
     s->hms[1] = t1 - t0;
-    free(s->hits);
-    s->nhits = nh;
-    s->hits = (accel_hit *) malloc(sizeof(accel_hit) * (nh ? nh : 1));
-    if (nh)
-        GPU(agpu_d2h(s->hits, s->d_hits, sizeof(agpu_hit) * nh, s->stream));
+    agpu_hitrec *all = rec + 1;
+    if (!rc && nh > first) {
+        agpu_hitrec *more = (agpu_hitrec *) realloc(rec, sizeof(agpu_hitrec) * ((size_t) nh + 1));
+        if (!more) {
+            set_err("out of host memory for %u hits", nh);
+            free(rec);
+            return -1;
+        }
+        rec = more;
+        all = rec + 1;
+        rc = agpu_d2h(all + first, s->d_hits + first, sizeof(agpu_hitrec) * (size_t) (nh - first),
+                      s->stream);
+    }
+    if (rc) {
+        set_err("collecting the hits: %s", agpu_last_error());
+        free(rec);
+        return -1;
+    }
     t0 = now_ms();
     s->hms[2] = t0 - t1;
-    int rc = replay(s);
+    free(s->hits);
+    free(s->sigs);
+    s->nhits = nh;
+    s->hits = (accel_hit *) malloc(sizeof(accel_hit) * (nh ? nh : 1));
+    s->sigs = (float *) malloc(sizeof(float) * (nh ? nh : 1));
+    rc = !s->hits || !s->sigs;
+    if (rc) {
+        s->nhits = 0;
+        set_err("out of host memory for %u hits", nh);
+    } else {
+        rc = sort_hits(all, nh);
+        for (unsigned i = 0; i < nh; i++) {
+            memcpy(&s->hits[i], &all[i].h, sizeof(accel_hit));
+            s->sigs[i] = all[i].sigma;
+        }
+    }
+    free(rec);
+    rc = rc ? -1 : replay(s);
     s->hms[3] = now_ms() - t0;
     return rc;
 }
@@ -2033,7 +2038,7 @@ long long accel_search_footprint(const accel_params *p)
     bytes += 24LL * (long long) (g.nblocks + 64) * (nfrac + 1); /* windows, norms */
     if (g.inmem)
         bytes += 4LL * ntiles * AGPU_TILE;                    /* per-half-bin norm^2 */
-    bytes += 24LL * HIT_CAP0;                                 /* hit buffer */
+    bytes += (long long) sizeof(agpu_hitrec) * HIT_CAP0;      /* hit buffer */
     bytes += 8LL * agpu_realfft_work(2 * g.numbins);          /* FFT work of series input */
     bytes += 64LL << 20;                                      /* refinement, tables, slack */
     if (g.numw)   /* jerk refinement scratch for a full chunk of candidates */

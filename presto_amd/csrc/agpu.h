@@ -30,6 +30,13 @@ typedef struct {
     float pow;   /* summed normalised power */
 } agpu_hit;
 
+/* A hit as the device keeps it, with its sigma (agpu_hit_sigmas). */
+typedef struct {
+    agpu_hit h;
+    float sigma;
+    int pad;
+} agpu_hitrec;
+
 /* Raw plane layout: tiles of AGPU_TILE half-bins, each tile holding every
  * (w,z) row contiguously, each tile-row followed by a halo of AGPU_HALO
  * half-bins that repeats the start of the same row in the next tile.
@@ -84,7 +91,7 @@ typedef struct {
     const float *nsq;        /* standard: [nblocks][nfrac+1]; in-memory: [npre+nblocks] */
     const float *nsq_hb;     /* in-memory: norm^2 for every half-bin [0, hb_end) */
     int npre;                /* in-memory pre-population blocks (start at half-bin 16) */
-    agpu_hit *hits;
+    agpu_hitrec *hits;
     unsigned int *nhits;
     unsigned int cap;
     /* address tables (agpu_harmsum_row_table / agpu_harmsum_chunk_tables) */
@@ -92,6 +99,14 @@ typedef struct {
     const long long *chunk_base;   /* [nchunks][AGPU_HS_CT] */
     const int *chunk_lo;           /* [nchunks][AGPU_HS_CT] */
 } agpu_harmsum_args;
+
+/* independent trials of each stage, for the sigmas */
+typedef struct {
+    double n[AGPU_MAX_STAGES];
+} agpu_numindep;
+/* sigma of the first min(*d_nhits, cap) hits, on the device */
+int agpu_hit_sigmas(agpu_hitrec *d_hits, const unsigned *d_nhits, unsigned cap,
+                    const agpu_numindep *ni, void *stream);
 
 /* Row table of the harmonic sum, per (w, z) row: [0] w index, [1] z index,
  * [AGPU_HS_RT_ROW] the row's offset in a tile (row x AGPU_ROWLEN floats),
