@@ -1924,7 +1924,7 @@ long accel_deredden_gpu(accel_fcomplex *fft, long long numbins, int startwidth, 
         agpu_h2d(d_blk, w, sizeof(agpu_window) * nb, stream) ||
         agpu_h2d(d_spec, fft, sizeof(accel_fcomplex) * (size_t) numbins, stream) ||
         agpu_deredden(d_spec, numbins, (const agpu_window *) d_blk, nb, maxn, (float *) d_mean,
-                      stream) ||
+                      0.0f, stream) ||
         agpu_d2h(fft, d_spec, sizeof(accel_fcomplex) * (size_t) numbins, stream)) {
         set_err("accel_deredden_gpu: %s", agpu_last_error());
         goto done;
@@ -1993,16 +1993,18 @@ static int set_series(accel_search *s, const float *series, long long n, int on_
     }
     /* realfft (src/accel_utils.c:1547), deredden (:1561), bin 0 := 1+1i
      * (:1621-1624; left as de-reddened under -photon), all on the device */
-    static const accel_fcomplex one = {1.0f, 1.0f};
-    if (on_device)
+    if (on_device) {
+        /* the caller's series is free once the copy is done; the rest runs on */
         GPU(agpu_copy_d2d(s->d_spec, series, sizeof(float) * (size_t) n, s->stream));
-    else
+        GPU(agpu_event_record(s->ev_norms, s->stream));
+    } else {
         GPU(agpu_h2d(s->d_spec, series, sizeof(float) * (size_t) n, s->stream));
+    }
     GPU(agpu_realfft((const float *) s->d_spec, n, s->d_spec, s->d_fftwork, s->stream));
     GPU(agpu_deredden(s->d_spec, g->numbins, s->d_dblk, s->ndblk, s->dmaxn, s->d_dmean,
-                      s->stream));
-    if (!(s->p.nph > 0.0))
-        GPU(agpu_h2d(s->d_spec, &one, sizeof(one), s->stream));
+                      s->p.nph > 0.0 ? 0.0f : 1.0f, s->stream));
+    if (on_device)
+        GPU(agpu_event_sync(s->ev_norms));
     return 0;
 }
 

@@ -148,6 +148,7 @@ int agpu_stream_wait_event(void *s, void *e);
 int agpu_event_create(void **e);
 int agpu_event_destroy(void *e);
 int agpu_event_record(void *e, void *stream);
+int agpu_event_sync(void *e);
 int agpu_event_elapsed(float *ms, void *start, void *stop);
 
 /* FP64 response templates for one segment length L (power of two):
@@ -257,9 +258,10 @@ int agpu_inmem_nsq_table(const float *d_nsq, int npre, int nblocks, long long rh
 
 /* De-reddening of a device spectrum in place (src/misc_utils.c:912-1067):
  * d_blk = the reference's median blocks {first bin, length} tiling
- * [1, numbins), maxn = the longest; d_mean receives nblk floats. */
+ * [1, numbins), maxn = the longest; d_mean receives nblk floats.  Bin 0
+ * becomes (1, im0). */
 int agpu_deredden(void *d_spec, long long numbins, const agpu_window *d_blk, int nblk,
-                  int maxn, float *d_mean, void *stream);
+                  int maxn, float *d_mean, float im0, void *stream);
 
 /* Complex values of work agpu_realfft and agpu_realfft_inverse need for
  * an n-sample series. */
