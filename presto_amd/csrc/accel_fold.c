@@ -258,13 +258,11 @@ int accel_fold_search(const double *rawfolds, const accel_foldstats *parts, int 
     const int npdd = searchpdd && !nosearch ? nt : 1;
     const size_t ncube = (size_t) npdd * nt * nt;
     double *fdotdots = (double *) malloc(sizeof(double) * nt);
-    double *pp = (double *) malloc(sizeof(double) * ncube);
     double *prof = (double *) malloc(sizeof(double) * proflen);
-    if (!periods || !fdots || !fdotdots || !pp || !prof) {
+    if (!periods || !fdots || !fdotdots || !prof) {
         free(periods);
         free(fdots);
         free(fdotdots);
-        free(pp);
         free(prof);
         accel_set_error("fold search: out of host memory");
         return -1;
@@ -291,14 +289,19 @@ int accel_fold_search(const double *rawfolds, const accel_foldstats *parts, int 
     st.numprof = proflen;
     int bip = (nt - 1) / 2, bipd = (nt - 1) / 2, bipdd = searchpdd ? (nt - 1) / 2 : 0, rc = -1;
     void *stream = NULL, *d_prof = NULL, *d_fd = NULL, *d_pt = NULL, *d_pp = NULL;
-    void *d_fdd = NULL;
+    void *d_fdd = NULL, *d_ppf = NULL, *d_first = NULL, *d_tmax = NULL;
     if (!nosearch) {
         const size_t pbytes = sizeof(double) * (size_t) npart * proflen;
+        const int tile = agpu_fold_tile(npart, proflen);
+        const size_t tiles = (size_t) ((nt + tile - 1) / tile);
+        unsigned long long first;
         if (agpu_init(device) || agpu_stream_create(&stream) || agpu_malloc(&d_prof, pbytes) ||
             agpu_malloc(&d_fd, sizeof(double) * nt) ||
             agpu_malloc(&d_pt, sizeof(double) * npart) ||
             agpu_malloc(&d_fdd, sizeof(double) * nt) ||
             agpu_malloc(&d_pp, sizeof(double) * ncube) ||
+            agpu_malloc(&d_ppf, sizeof(float) * ncube) || agpu_malloc(&d_first, sizeof(first)) ||
+            agpu_malloc(&d_tmax, sizeof(first) * (ncube / nt) * tiles) ||
             agpu_h2d(d_prof, rawfolds, pbytes, stream) ||
             agpu_h2d(d_fd, fdots, sizeof(double) * nt, stream) ||
             agpu_h2d(d_fdd, fdotdots, sizeof(double) * nt, stream) ||
@@ -320,30 +323,27 @@ int accel_fold_search(const double *rawfolds, const accel_foldstats *parts, int 
         for (int ipdd = 0; ipdd < npdd; ipdd++) {
             a.ipdd = ipdd;
             a.redchi = (double *) d_pp + (size_t) ipdd * nt * nt;
+            a.redchif = (float *) d_ppf + (size_t) ipdd * nt * nt;
+            a.tilemax = (unsigned long long *) d_tmax + (size_t) ipdd * nt * tiles;
             if (agpu_fold_search(&a, stream)) {
                 accel_set_error("fold search: %s", agpu_last_error());
                 goto done;
             }
         }
-        if (agpu_d2h(pp, d_pp, sizeof(double) * ncube, stream) || agpu_stream_sync(stream)) {
+        /* the plane as floats, as the reference keeps it, and the first
+         * maximum in (p-dotdot, p-dot, period) order: the reference's
+         * strictly-greater test over its loops, from a redchi of 0 */
+        if (agpu_fold_first((const double *) d_pp, (const unsigned long long *) d_tmax,
+                            ncube / nt, nt, tile, (unsigned long long *) d_first, stream) ||
+            agpu_d2h(&first, d_first, sizeof(first), stream) ||
+            (ppdot && agpu_d2h(ppdot, d_ppf, sizeof(float) * ncube, stream))) {
             accel_set_error("fold search: %s", agpu_last_error());
             goto done;
         }
-        /* the first maximum in (p-dotdot, p-dot, period) order: the
-         * reference's strictly-greater test over its loops, from a redchi
-         * of 0 */
-        double bestrc = 0.0;
-        bip = bipd = bipdd = 0;
-        for (size_t i = 0; i < ncube; i++)
-            if (pp[i] > bestrc) {
-                bestrc = pp[i];
-                bip = (int) (i % nt);
-                bipd = (int) (i / nt % nt);
-                bipdd = (int) (i / ((size_t) nt * nt));
-            }
-        if (ppdot)   /* float, as the reference keeps its plane */
-            for (size_t i = 0; i < ncube; i++)
-                ppdot[i] = (float) pp[i];
+        const size_t i = (size_t) first;
+        bip = (int) (i % nt);
+        bipd = (int) (i / nt % nt);
+        bipdd = (int) (i / ((size_t) nt * nt));
     }
     /* the best profile and its statistics (the redchi in FP64, as
      * combine_profs leaves it) */
@@ -372,13 +372,15 @@ done:
     agpu_free(d_fd);
     agpu_free(d_pt);
     agpu_free(d_pp);
+    agpu_free(d_ppf);
+    agpu_free(d_first);
+    agpu_free(d_tmax);
     agpu_free(d_fdd);
     if (stream)
         agpu_stream_destroy(stream);
     free(periods);
     free(fdots);
     free(fdotdots);
-    free(pp);
     free(prof);
     return rc;
 }

@@ -372,8 +372,19 @@ typedef struct {
     int npart, proflen, numtrials, pstep;
     int ipdd;             /* the p-dotdot trial of this launch (with fdotdots) */
     double *redchi;       /* numtrials x numtrials, [ipd][ip], of trial ipdd */
+    float *redchif;       /* the same, rounded */
+    /* per tile of agpu_fold_tile consecutive periods, [ipd][tile]: the bits
+     * of its largest redchi above 0, or 0 */
+    unsigned long long *tilemax;
 } agpu_fold_search_args;
 int agpu_fold_search(const agpu_fold_search_args *args, void *stream);
+/* periods per tile of the search */
+int agpu_fold_tile(int npart, int proflen);
+/* *d_first := the smallest index of the largest redchi above 0 of rows x
+ * numtrials trials, 0 if there is none */
+int agpu_fold_first(const double *d_redchi, const unsigned long long *d_tilemax,
+                    unsigned long long rows, int numtrials, int tile,
+                    unsigned long long *d_first, void *stream);
 
 #ifdef __cplusplus
 }

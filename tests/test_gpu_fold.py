@@ -205,3 +205,32 @@ def test_gpu_fold_search_pdotdot_equals_oracle(npart, nb, fdd):
     assert (best.ip, best.ipd, best.ipdd) == (wb["ip"], wb["ipd"], wb["ipdd"])
     assert best.p == wb["p"] and best.pd == wb["pd"] and best.pdd == wb["pdd"]
     assert best.stats.redchi == pytest.approx(wb["redchi"], rel=1e-13)
+
+
+@pytest.mark.parametrize("npart,nb,npfact,flat", [
+    (1, 2, 1, False),      # five periods, one part
+    (9, 15, 1, False),     # 31 periods: a tile less one
+    (8, 16, 1, False),     # 33: a tile and one period
+    (64, 73, 1, False),    # the most bins whose tile fits the LDS for 64 parts
+    (64, 74, 1, False),    # one more: a workgroup per trial
+    (4, 16, 1, True),      # no redchi above 0: the first trial
+])
+def test_gpu_fold_search_tiles(npart, nb, npfact, flat):
+    """The edges of the search's tiles, with noise in the folds: plane and
+    best trial as the oracle's, bit for bit."""
+    _say(f"case: fold search tiles npart={npart} proflen={nb} npfact={npfact} flat={flat}")
+    N, dt, f = 1 << 17, 1e-3, 5.1
+    x = synth.make_series(N, dt, 31, [dict(f0=f, z=0.0, duty=0.2, amp=0.2)])
+    prof, parts, total, n = A.fold(x, dt, f, 0.0, 0.0, npart=npart, proflen=nb)
+    st = [{k: getattr(p, k) for k, _ in A.FoldStats._fields_} for p in parts]
+    if flat:
+        for p, s in zip(parts, st):
+            prof[:] = 1.0
+            p.prof_avg = s["prof_avg"] = 1.0
+    pt = _parttimes(N, dt, npart)
+    pp, _, best = A.fold_search(prof, parts, f, 0.0, 0.0, n * dt, pt, npfact=npfact)
+    want, wb = O.fold_search(prof, st, f, 0.0, 0.0, n * dt, pt, npfact=npfact)
+    assert pp.shape == want.shape == (2 * npfact * nb + 1,) * 2
+    assert np.array_equal(pp.view(np.uint32), want.view(np.uint32))
+    assert (best.ip, best.ipd) == (wb["ip"], wb["ipd"])
+    assert not flat or (best.ip, best.ipd) == (0, 0) and not pp.any()
