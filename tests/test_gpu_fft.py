@@ -68,3 +68,20 @@ def test_search_on_a_non_power_of_two_series(N, dt):
     for g, w in zip(cands, want):
         assert g["numharm"] == int(w[2]) and abs(g["r"] - w[3]) < 1e-3
         assert abs(g["z"] - w[4]) < 0.05 and abs(g["sigma"] - w[1]) < 1e-3
+
+
+@pytest.mark.parametrize("M", [64, 64 * 3, 64 * 27, 64 * 33, 64 * 2, 64 * 64, 64 * 64 * 4 * 3,
+                               64 * 64 * 8 * 13, 64 * 64 * 64 * 5])
+def test_paired_passes(M):
+    """Lengths whose powers of two run as pairs of radix-8 passes: a part of
+    one workgroup's 32 columns, one column more than a workgroup, several
+    pairs, each radix that can follow.  Every output is a sum over 3 log2(M)
+    roundings or so of values of its own rms; 8 log2(n) units of 2^-24 leave
+    room for the largest bin."""
+    n = 2 * M
+    print(f"case: realfft pairs M={M}", flush=True)
+    x = np.random.default_rng(M).standard_normal(n).astype(np.float32)
+    bar = 8 * np.log2(n) * 2.0 ** -24
+    err, dc, ny = _rms_err(A.realfft_gpu(x), x)
+    print(f"  worst bin / rms {err:.2e}, bound {bar:.2e}", flush=True)
+    assert err < bar
