@@ -13,11 +13,15 @@ GPU figures are comparable; DM-trials/s and p50/p99 step latency are
 reported beside it.
 
 Roofline: per-kernel durations come from HIP events recorded on the
-search's own stream around each launch.  Algorithmic bytes per fundamental
-cell (the reference geometry's cells): harmonic sum 4 (1 + sum_f (k/H)^2)
-bytes (the fundamental plus each sub-harmonic fraction's share of the
-plane), correlation 4 bytes per raw-plane cell written plus the spectrum
-and template reads.  `traffic` is the measured HBM bytes per launch from
+search's own stream around each launch.  `roofline` is the longest kernel's,
+the correlation's, against its bound, the FP32 vector rate: per segment and
+template two inverse 2048-point transforms (5 N log2 N each), the products
+with the spectrum and |.|^2 of the kept outputs, plus a forward transform
+per segment and template group.  `roofline_harmonic_sum`: the harmonic sums
+by bounds read half a byte per fundamental cell (a 16-bit bound for every 4
+half-bins) and as much of the sub-harmonic fractions' shares, 0.5 (1 +
+sum_f (k/H)^2) bytes in all, an eighth of what summing every cell reads
+(`every_cell_bytes`).  `traffic` is the measured HBM bytes per launch from
 the committed rocprofv3 counter summary profiles/plain_2e23_counters.md
 (FETCH_SIZE x 2 + WRITE_SIZE, the scale of a plain copy kernel).
 `hbm_read_ceiling` is what a streaming-read kernel (k_read_probe, 16-byte
@@ -517,18 +521,21 @@ def main():
     cells = g.nblocks * g.corr_uselen * g.numz * numw
     ms_step = 1e3 * wall / args.steps
     nfrac = [(k, 1 << st) for st in range(1, g.numharmstages) for k in range(1, 1 << st, 2)]
-    hs_bytes_per_cell = 4.0 * (1.0 + sum((k / h) ** 2 for k, h in nfrac))
-    hs_bytes = hs_bytes_per_cell * cells
+    hs_share = 1.0 + sum((k / h) ** 2 for k, h in nfrac)
+    hs_bytes = 0.5 * hs_share * cells
     hs_ms = avg("harmsum")
     corr_ms = avg("corr")
     nt = g.numz * numw
-    corr_bytes = 4.0 * plane_cells + 8.0 * g.numbins + 8.0 * nt * shape["L"]
+    # written: the plane and a 16-bit bound for every 4 half-bins
+    corr_bytes = 4.5 * plane_cells + 8.0 * g.numbins + 8.0 * nt * shape["L"]
     L, U = shape["L"], shape["uselen"]
-    fft_flops = 5.0 * L * np.log2(L)
-    # per (segment, template): inverse FFT, spectrum x template, |.|^2 of the
-    # kept outputs; per (segment, template group): the forward FFT
-    corr_flops = shape["nseg"] * (nt * (fft_flops + 6.0 * L + 3.0 * U)
+    fft_flops = 5.0 * (L / 2) * np.log2(L / 2)
+    # per (segment, template): two half-length inverse FFTs, spectrum x
+    # template, |.|^2 of the kept outputs; per (segment, template group): the
+    # forward FFT of the segment's bins
+    corr_flops = shape["nseg"] * (nt * (2.0 * fft_flops + 6.0 * L + 3.0 * U)
                                   + shape["groups"] * fft_flops)
+    corr_tflops = corr_flops / (corr_ms * 1e-3) / 1e12
 
     line = {
         "metric": METRIC,
@@ -561,23 +568,25 @@ def main():
         "host_ms": {k: float(np.mean([h[k] for h in host])) for k in host[0]},
         "candidates": ncand,
         "hits": nhits,
-        "roofline": {"bound": "hbm", "kernel": "k_harmsum<5,0>",
-                     "achieved": hs_bytes / (hs_ms * 1e-3) / 1e9, "peak": HBM_PEAK_GBS,
-                     "unit": "GB/s",
-                     "frac": hs_bytes / (hs_ms * 1e-3) / 1e9 / HBM_PEAK_GBS,
-                     "traffic": measured_traffic("k_harmsum<5, 0>"),
-                     "bytes_per_cell": hs_bytes_per_cell,
-                     "frac_of_read_ceiling": (hs_bytes / (hs_ms * 1e-3) / 1e9 / ceiling["gbs"]
-                                              if ceiling else None)},
+        "roofline": {"bound": "valu", "kernel": "k_corr<true>",
+                     "achieved": corr_tflops, "peak": VALU_PEAK_TFLOPS, "unit": "TFLOP/s",
+                     "frac": corr_tflops / VALU_PEAK_TFLOPS,
+                     "achieved_gbs": corr_bytes / (corr_ms * 1e-3) / 1e9,
+                     "hbm_frac": corr_bytes / (corr_ms * 1e-3) / 1e9 / HBM_PEAK_GBS,
+                     "traffic": measured_traffic("k_corr<true>")},
+        "roofline_harmonic_sum": {"bound": "issue", "kernel": "k_harmbound<5, 0>",
+                                  "achieved": hs_bytes / (hs_ms * 1e-3) / 1e9,
+                                  "peak": HBM_PEAK_GBS, "unit": "GB/s",
+                                  "frac": hs_bytes / (hs_ms * 1e-3) / 1e9 / HBM_PEAK_GBS,
+                                  "traffic": measured_traffic("k_harmbound<5, 0>"),
+                                  "bytes_per_cell": 0.5 * hs_share,
+                                  "every_cell_bytes": 4.0 * hs_share,
+                                  "frac_of_read_ceiling":
+                                      (hs_bytes / (hs_ms * 1e-3) / 1e9 / ceiling["gbs"]
+                                       if ceiling else None)},
         "hbm_read_ceiling": ceiling,
         "corr_tuning": {"groups_kept": tuned[0],
                         "timed_groups_ms": tuned[1]},
-        "roofline_correlation": {"bound": "valu", "kernel": "k_corr4096",
-                                 "achieved_gbs": corr_bytes / (corr_ms * 1e-3) / 1e9,
-                                 "hbm_frac": corr_bytes / (corr_ms * 1e-3) / 1e9 / HBM_PEAK_GBS,
-                                 "achieved_tflops": corr_flops / (corr_ms * 1e-3) / 1e12,
-                                 "valu_peak_tflops": VALU_PEAK_TFLOPS,
-                                 "traffic": measured_traffic("k_corr4096")},
     }
     if args.batch_trials > 0:
         line["batched"] = batched_section(args.batch_trials, args.cpu_threads)

@@ -158,7 +158,7 @@ int accel_search_nwindows(const accel_search *s);
 int accel_search_norms(const accel_search *s, double *out, int n);
 /* Milliseconds of the last run (HIP events): block norms (on a second
  * stream, beside the correlation), correlation, the gap between the
- * correlation and the harmonic sum (the plane's tile halos are written by
+ * correlation and the harmonic sum (the plane's halos or bounds are written by
  * the correlation, so about 0), harmonic sum (including any wait for the
  * norms), total. */
 int accel_search_timings(const accel_search *s, float *ms5);

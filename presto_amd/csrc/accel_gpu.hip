@@ -743,7 +743,7 @@ __device__ __forceinline__ void fft2048_mid(float2 *v, float2 *buf, int j, const
  * template (196 for the template product and the first radix 16, 192, 144,
  * 32 for the powers) and ~80 for the stores, against ~760 for one
  * 4096-point transform with separate twiddle products: 2.0 ms of issue for
- * the 2^23-sample, zmax 200 search, measured 2.87 ms beside the norms
+ * the 2^23-sample, zmax 200 search, measured 2.7 ms beside the norms
  * (3.91 ms before; 2^20 samples, 201 x 31 templates: 10.6 ms, 14.1 ms).
  * 124 VGPRs and 35 KB of LDS: four workgroups per CU, against two. */
 template <bool BOUNDS>
@@ -1604,9 +1604,9 @@ __device__ __forceinline__ void hb_add_stage(float *acc, const unsigned *lds, co
  * the same for every row and chunk: the inner loop is LDS reads, maxima and
  * multiply-adds without any index arithmetic.
  *
- * 2^23 samples, zmax 200, 16 harmonics: 2.1 ms against k_harmsum's 7.4 (1/8
+ * 2^23 samples, zmax 200, 16 harmonics: 1.85 ms against k_harmsum's 7.4 (1/8
  * of its 39 GB; 1.3 % of the 64-cell runs summed exactly); 2^20, 201 x 31
- * templates, 8 harmonics: 3.1 ms against 14.4.  Bound: vector and scalar
+ * templates, 8 harmonics: 2.5 ms against 14.4.  Bound: vector and scalar
  * issue (1.1 ms of it) and the latency of the two load-store-sum phases at
  * four waves per SIMD. */
 template <int NSTAGES, int MODE>

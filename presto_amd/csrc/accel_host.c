@@ -8,9 +8,11 @@
  *
  * Device layout (one search):
  *   spectrum   float2[numbins]                       (bin lobin first)
- *   templates  float2[numw'][numz][L]                L = 4096, FP32, 1/L folded in
- *   raw plane  float, tiles of 2048 half-bins x every  column = absolute half-bin,
- *              (w,z) row (AGPU_PLANE_IDX)             un-normalised |corr|^2
+ *   templates  float2[numw'][numz][L]                L = 4096, FP32, 1/L folded in:
+ *              the even and the odd half-bins' 2048-point templates
+ *   raw plane  float, tiles of 8192 half-bins x every  column = absolute half-bin,
+ *              (w,z) row (AGPU_PLANE_IDX), behind     un-normalised |corr|^2
+ *              each tile-row its halo or its bounds
  *   windows    {lobin, numdata}[nwin] -> norm (FP64), nsq = norm^2 (FP32)
  *   zmap/wmap  int[nfrac][numz] / int[nfrac][numw']  sub-harmonic rows
  *   hits       counter + agpu_hitrec[cap] (hit, sigma)
@@ -912,7 +914,7 @@ int accel_search_launch(accel_search *s)
                        s->hb_end, s->d_plane, s->ntiles, s->groups, 0, -1, s->bounds,
                        s->stream));
     GPU(agpu_event_record(s->ev[2], s->stream));
-    /* the tile halos are written by the correlation itself */
+    /* the tile halos or bounds are written by the correlation itself */
     GPU(agpu_event_record(s->ev[3], s->stream));
     if (two)
         GPU(agpu_stream_wait_event(s->stream, s->ev_norms));
