@@ -1604,11 +1604,13 @@ __device__ __forceinline__ void hb_add_stage(float *acc, const unsigned *lds, co
  * the same for every row and chunk: the inner loop is LDS reads, maxima and
  * multiply-adds without any index arithmetic.
  *
- * 2^23 samples, zmax 200, 16 harmonics: 1.85 ms against k_harmsum's 7.4 (1/8
- * of its 39 GB; 1.3 % of the 64-cell runs summed exactly); 2^20, 201 x 31
- * templates, 8 harmonics: 2.5 ms against 14.4.  Bound: vector and scalar
- * issue (1.1 ms of it) and the latency of the two load-store-sum phases at
- * four waves per SIMD. */
+ * 2^23 samples, zmax 200, 16 harmonics: 1.85 ms against k_harmsum's 7.4 (an
+ * eighth of its 39 GB needed; 1.3 % of the 64-cell runs summed exactly);
+ * 2^20, 201 x 31 templates, 8 harmonics: 2.5 ms against 14.4.  Bound: vector
+ * and scalar issue (1.1 ms of it) and the latency of the two load-store-sum
+ * phases at four waves per SIMD.  Chunks on other XCDs share the cache lines
+ * of a sub-harmonic's bounds (12.3 GB fetched for 4.9); runs of 32 chunks per
+ * XCD halve that and leave whole searches between 2 % slower and 1 % faster. */
 template <int NSTAGES, int MODE>
 __global__ __launch_bounds__(256) void k_harmbound(agpu_harmsum_args a, const float *nb,
                                                    int chunks, int zblocks, int zrows)
@@ -2263,14 +2265,17 @@ int agpu_harmsum(const agpu_harmsum_args *a, long long c_lo, long long c_hi, voi
 /* Bounds pay
  *  - while few cells pass them: on whitened noise the bound of a sum of H
  *    powers is 2.13 H on average (the largest of 4 half-bins, or of 4 and 4)
- *    with a spread of 1.3 sqrt(H); with a threshold 2.4 spreads up a tenth
+ *    with a spread of 1.3 sqrt(H); with a threshold 2.3 spreads up a tenth
  *    of the 64-cell runs are summed exactly.  16 harmonics, 2^18 samples,
- *    zmax 100 (3.0 sqrt(H) up): 130 us against k_harmsum's 118; 2^19, zmax
- *    100 (3.3): 151 against 219; 2^21, zmax 100 (3.8): 341 against 1100;
+ *    zmax 100 (3.0 sqrt(H) up): 88 us against k_harmsum's 118; 2^19, zmax
+ *    100 (3.3): 123 against 232; 2^21, zmax 100 (3.8): 345 against 1133.  The
+ *    line is above the first: a spectrum's lines cross there before noise does
+ *    (one every 32 bins, 2^23 samples, zmax 200: 5.3 ms against 4.3);
  *  - with rows for the lanes and workgroups for the device: 8 harmonics,
- *    2^21 samples, 5 rows 58 us against 37, 11 rows 60 against 62, 21 rows
- *    62 against 107; 21 rows of 2^18 half-bins 28 against 24, of 2^19 31
- *    against 36, 51 rows of 2^18 34 against 40. */
+ *    2^21 samples, 5 rows 54 us against 37, 11 rows 56 against 62 (whole
+ *    search 175 either way), 21 rows 59 against 105; 21 rows of 2^18
+ *    half-bins 37 against 23, of 2^19 37 against 35, 51 rows of 2^18 43
+ *    against 40: near 2^23 cells the two are alike. */
 int agpu_harmbound_pays(int nstages, const float *powcut, int corr_uselen, int numz, int numw,
                         long long numhb, int nfrac, const int *zmap)
 {
