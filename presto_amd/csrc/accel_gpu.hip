@@ -1355,6 +1355,24 @@ __global__ void k_bound_norms(agpu_harmsum_args a, int c0, int nc, long long hb_
     nb[(size_t) c * 32 + f] = m + m * 0x1p-18f;
 }
 
+/* Bounds at and past hb_end, which k_corr does not write: 0.  The chunk that
+ * holds the last half-bin looks at them beside the bounds before hb_end, in
+ * one maximum over a lane's 16 sums, so what an earlier user left in the
+ * memory must not stand there (the bits of a negative sum exceed those of
+ * every power and would hide the lane's other sums).  Once per plane:
+ * nothing writes them later.  first: the first tile with such a slot, of its
+ * own or of the next tile's first groups. */
+__global__ __launch_bounds__(256) void k_clear_bounds(float *plane, long long tile_stride,
+                                                      long long hb_end, long long first)
+{
+    const long long tile = first + blockIdx.y;
+    unsigned short *b = (unsigned short *) (plane + tile * tile_stride +
+                                            (long long) blockIdx.x * AGPU_ROWLEN + AGPU_TILE);
+    for (int i = threadIdx.x; i < AGPU_TILE / AGPU_GROUP + AGPU_BHALO; i += 256)
+        if (tile * AGPU_TILE + (long long) i * AGPU_GROUP >= hb_end)
+            b[i] = 0;
+}
+
 /* Exact sums of 64 cells, lane l at fundamental half-bin hb + l, of every
  * z row z0 + i with bit i set in todo (not 0), straight from the raw plane:
  * the terms and their order are k_harmsum's.  The lanes of a fraction lie
@@ -2308,6 +2326,18 @@ long long agpu_harmbound_chunks(const agpu_harmsum_args *a)
 {
     const long long ncell = (long long) a->nblocks * a->corr_uselen;
     return ncell > 0 ? (a->rh0 + ncell - 1) / HB_CHUNK - a->rh0 / HB_CHUNK + 1 : 0;
+}
+
+int agpu_clear_bounds(float *d_plane, int nrows, long long ntiles, long long hb_end, void *stream)
+{
+    const long long own = hb_end >> AGPU_TILE_LOG2, first = own > 0 ? own - 1 : 0;
+    if (!d_plane || nrows < 1 || hb_end < 0 || first >= ntiles || ntiles - first > 65535)
+        return fail("agpu_clear_bounds: bad plane");
+    hipLaunchKernelGGL(k_clear_bounds, dim3((unsigned) nrows, (unsigned) (ntiles - first)),
+                       dim3(256), 0, (hipStream_t) stream, d_plane,
+                       (long long) nrows * AGPU_ROWLEN, hb_end, first);
+    AGPU_CHECK(hipGetLastError());
+    return 0;
 }
 
 int agpu_bound_norms(const agpu_harmsum_args *a, long long hb_end, float *d_nb, void *stream)

@@ -758,7 +758,8 @@ static int search_init(accel_search *s, int device, int nstreams)
         agpu_harmsum_args a;
         fill_harmsum_args(s, &a);
         const long long nc = agpu_harmbound_chunks(&a);
-        rc = agpu_malloc((void **) &s->d_nb, sizeof(float) * 32 * (size_t) (nc > 0 ? nc : 1));
+        rc = agpu_malloc((void **) &s->d_nb, sizeof(float) * 32 * (size_t) (nc > 0 ? nc : 1)) ||
+             agpu_clear_bounds(s->d_plane, s->nt, s->ntiles, s->hb_end, s->stream);
     }
     free(rowtab);
     free(cbase);

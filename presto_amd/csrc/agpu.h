@@ -248,6 +248,9 @@ long long agpu_harmsum_nchunks(const agpu_harmsum_args *a);
 int agpu_harmbound_pays(int nstages, const float *powcut, int corr_uselen, int numz, int numw,
                         long long numhb, int nfrac, const int *zmap);
 long long agpu_harmbound_chunks(const agpu_harmsum_args *a);
+/* Once per plane, before its first search by bounds: the bounds at and past
+ * hb_end, which no correlation writes and the last chunk reads, become 0. */
+int agpu_clear_bounds(float *d_plane, int nrows, long long ntiles, long long hb_end, void *stream);
 int agpu_bound_norms(const agpu_harmsum_args *a, long long hb_end, float *d_nb, void *stream);
 int agpu_harmbound(const agpu_harmsum_args *a, const float *d_nb, void *stream);
 long long agpu_harmsum_chunk_hb(const agpu_harmsum_args *a, long long c);

@@ -5,6 +5,8 @@ The shapes are those at which it can go wrong: 1 to 5 stages, both index
 rules, row blocks below, at and above 64 rows, jerk rows, ragged lengths, a
 first half-bin off every chunk edge, strong signals, bins without power,
 infinities and NaN."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -108,3 +110,45 @@ def test_hits_equal_the_sums(nbins, zmax, wmax, numharm, inmem, rlo, odd):
     assert len(want) > 20
     assert [h[:5] for h in got] == [h[:5] for h in want]
     np.testing.assert_array_equal(np.array([h[5] for h in got]), np.array([h[5] for h in want]))
+
+
+@pytest.fixture
+def used_memory():
+    """Device memory whose last user left a large negative number in every
+    word (0xfefe...): an arena, as the request loop's handles share one."""
+    lib, n, p = A.lib, 1 << 30, C.c_void_p()
+    lib.agpu_malloc.argtypes = [C.c_void_p, C.c_size_t]
+    lib.agpu_memset.argtypes = [C.c_void_p, C.c_int, C.c_size_t, C.c_void_p]
+    lib.agpu_free.argtypes = lib.agpu_stream_sync.argtypes = [C.c_void_p]
+    lib.agpu_arena_init.argtypes = [C.c_size_t]
+    lib.accel_template_cache_clear()
+    assert lib.agpu_init(0) == 0 and lib.agpu_arena_init(n) == 0
+    assert lib.agpu_malloc(C.byref(p), n) == 0 and lib.agpu_memset(p, 0xfe, n, None) == 0
+    assert lib.agpu_stream_sync(None) == 0 and lib.agpu_free(p) == 0
+    yield
+    lib.accel_template_cache_clear()
+    assert lib.agpu_arena_release() == 0
+
+
+@pytest.mark.parametrize("numharm,inmem", [(1, False), (8, True), (16, False)])
+def test_the_last_half_bins_in_used_memory(used_memory, numharm, inmem):
+    """A signal in the last, partial run of 64 half-bins, whose other bounds
+    no correlation writes."""
+    nbins, rlo = (150000, 110) if numharm < 16 else (1 << 18, 77)
+    p = A.make_params(nbins, 2 * nbins, 1e-3, zmax=30 if numharm < 16 else 100, numharm=numharm,
+                      sigma=2.5, rlo=rlo, rhi=nbins - 1, inmem=inmem, force_standard=not inmem,
+                      dat_input=False)
+    g = A.geometry(p)
+    end = 2 * int(np.floor(np.rint(2 * g.rlo) / 2)) + g.nblocks * g.corr_uselen
+    run = end // 64 * 64
+    assert 16 <= end - run <= 48
+    with A.Search(p) as s:
+        assert _by_bounds(s.geom)
+        s.set_spectrum(_spectrum(nbins, 5, [(run // 2 + 2, 40.0)]))
+        s.run()
+        got = [(int(h["block"]), int(h["stage"]), int(h["wi"]), int(h["zi"]), int(h["ii"]),
+                h["pow"]) for h in s.hits()]
+        want = _expected(s)
+    assert sum(h[0] * g.corr_uselen + h[4] + end - g.nblocks * g.corr_uselen >= run
+               for h in want) > 5
+    assert got == want
