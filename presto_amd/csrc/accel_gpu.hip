@@ -901,7 +901,9 @@ __global__ __launch_bounds__(256, 4) void k_corr(const float2 *spec, long long n
         if (BOUNDS) {
             /* the group's largest power rounded up to 16 bits: an upper bound
              * that the harmonic sum looks at before it reads the powers.  Bit
-             * patterns, which order like the powers: a NaN stays one */
+             * patterns, which order like the powers.  A NaN, whose bits reach
+             * up to ~0u, must not carry out of the rounding: any above
+             * 0x7fff0000 becomes the positive NaN 0x7fff */
             int e = eg;
             asm volatile("" : "+v"(e));   /* see below */
 #pragma unroll
@@ -914,7 +916,7 @@ __global__ __launch_bounds__(256, 4) void k_corr(const float2 *spec, long long n
                     w[h] = max(x, (unsigned) __builtin_amdgcn_update_dpp(
                                       0, (int) x, 0xb1 /* lanes 1,0,3,2 */, 0xf, 0xf, true));
                 }
-                const unsigned bnd = ((tid & 1 ? w[1] : w[0]) + 0xffffu) >> 16;
+                const unsigned bnd = (min(tid & 1 ? w[1] : w[0], 0x7fff0000u) + 0xffffu) >> 16;
                 store_bound(row, goff[m], bnd);
                 if (halo) {
                     const unsigned g = (unsigned) (e + 1024 * m) / AGPU_GROUP;

@@ -152,3 +152,32 @@ def test_the_last_half_bins_in_used_memory(used_memory, numharm, inmem):
     assert sum(h[0] * g.corr_uselen + h[4] + end - g.nblocks * g.corr_uselen >= run
                for h in want) > 5
     assert got == want
+
+
+@pytest.mark.parametrize("bits", [0x7fffffff, 0xffffffff, 0x7fc00000])
+def test_nan_beside_a_signal(bits):
+    """A NaN, whatever its payload and sign, fills one segment of the
+    correlation; the signal lies in the next one, in the same run of 64
+    half-bins."""
+    nbins = 150000
+    p = A.make_params(nbins, 2 * nbins, 1e-3, zmax=40, numharm=1, sigma=2.5, rlo=100,
+                      rhi=nbins - 1, force_standard=True, dat_input=False)
+    with A.Search(p) as s:
+        assert _by_bounds(s.geom)
+        uselen = s.corr_shape()["uselen"]
+        hw = (4096 - uselen) // 4
+        end = next(e for e in range(20 * uselen, 60 * uselen, uselen) if 16 <= e % 64 <= 48)
+        X = _spectrum(nbins, 6, [(end // 2 + 2, 40.0)])
+        bad = (end - uselen) // 2 + hw + 10   # in reach of no other segment
+        X.view(np.uint32)[2 * bad:2 * bad + 2] = bits
+        s.set_spectrum(X)
+        s.run()
+        got = [(int(h["block"]), int(h["stage"]), int(h["wi"]), int(h["zi"]), int(h["ii"]),
+                h["pow"]) for h in s.hits()]
+        want = _expected(s)
+        for z in range(s.geom.numz):
+            assert np.isnan(s.plane_row(0, z, end - 4, 4)).all()
+            assert np.isfinite(s.plane_row(0, z, end, 4)).all()
+    near = [h for h in want
+            if end <= 200 + h[0] * s.geom.corr_uselen + h[4] < (end // 64 + 1) * 64]
+    assert len(near) > 5 and got == want
