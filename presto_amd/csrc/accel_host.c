@@ -862,8 +862,14 @@ int accel_search_set_spectrum(accel_search *s, const accel_fcomplex *fft)
 
 int accel_search_set_device_spectrum(accel_search *s, const void *d_fft)
 {
-    if (s->own_spec)
-        agpu_free(s->d_spec);
+    if (s->own_spec) {
+        /* its preparation or a launched search may still be running, and an
+         * arena hands a freed block to the next handle at once */
+        GPU(agpu_stream_sync(s->stream));
+        if (s->stream2 != s->stream)
+            GPU(agpu_stream_sync(s->stream2));
+        GPU(agpu_free(s->d_spec));
+    }
     s->own_spec = 0;
     s->d_spec = (void *) d_fft;
     return 0;

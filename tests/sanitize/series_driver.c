@@ -1,0 +1,164 @@
+/*
+ * Host-only driver for what the series and spectrum setters of a search
+ * handle (accel_host.c, included here so that a handle can be laid out by
+ * hand) promise about memory and streams, built by tests/test_sanitize.py.
+ * The device layer is replaced by test doubles that only book: an operation
+ * stays pending on its stream, with the buffers it reads and writes, until
+ * the stream, or an event recorded behind it, is waited for.
+ *
+ * Exits 0 when every check holds.
+ */
+#include "accel_host.c"
+
+#define CHECK(c)                                                           \
+    do {                                                                   \
+        if (!(c)) {                                                        \
+            fprintf(stderr, "check failed: %s (line %d)\n", #c, __LINE__); \
+            exit(1);                                                       \
+        }                                                                  \
+    } while (0)
+
+/* ---- test doubles of the device layer ---- */
+
+static struct {
+    const void *stream, *rd, *wr;
+} g_op[64];
+static int g_nop;
+
+struct event {
+    const void *stream;
+    int mark;   /* operations enqueued before it */
+};
+
+static void op(const void *stream, const void *rd, const void *wr)
+{
+    CHECK(g_nop < 64);
+    g_op[g_nop].stream = stream;
+    g_op[g_nop].rd = rd;
+    g_op[g_nop++].wr = wr;
+}
+
+/* the first n operations of a stream are done */
+static int done(const void *stream, int n)
+{
+    for (int i = 0; i < n; i++)
+        if (g_op[i].stream == stream)
+            g_op[i].rd = g_op[i].wr = NULL;
+    return 0;
+}
+
+static int pending(const void *p)
+{
+    for (int i = 0; i < g_nop; i++)
+        if (g_op[i].rd == p || g_op[i].wr == p)
+            return 1;
+    return 0;
+}
+
+static const char *g_fail = "";   /* the double that fails */
+
+int agpu_malloc(void **p, size_t bytes) { return (*p = malloc(bytes)) == NULL; }
+int agpu_free(void *p)
+{
+    CHECK(!p || !pending(p));   /* an arena hands a freed block out at once */
+    free(p);
+    return 0;
+}
+int agpu_h2d(void *dst, const void *src, size_t bytes, void *stream)
+{
+    (void) dst, (void) src, (void) bytes;
+    return done(stream, g_nop);
+}
+int agpu_copy_d2d(void *dst, const void *src, size_t bytes, void *stream)
+{
+    (void) bytes;
+    op(stream, src, dst);
+    return 0;
+}
+int agpu_stream_sync(void *stream) { return done(stream, g_nop); }
+int agpu_event_record(void *e, void *stream)
+{
+    ((struct event *) e)->stream = stream;
+    ((struct event *) e)->mark = g_nop;
+    return 0;
+}
+int agpu_event_sync(void *e)
+{
+    return done(((struct event *) e)->stream, ((struct event *) e)->mark);
+}
+const char *agpu_last_error(void) { return "double"; }
+long long agpu_realfft_work(long long n) { return n; }
+int agpu_realfft(const float *x, long long n, void *out, void *work, void *stream)
+{
+    (void) n, (void) work;
+    if (!strcmp(g_fail, "realfft"))
+        return -1;
+    op(stream, x, out);
+    return 0;
+}
+int agpu_deredden(void *spec, long long numbins, const agpu_window *blk, int nblk, int maxn,
+                  float *mean, float im0, void *stream)
+{
+    (void) numbins, (void) blk, (void) nblk, (void) maxn, (void) mean, (void) im0;
+    op(stream, spec, spec);
+    return 0;
+}
+
+/* ---- a handle with what the setters use ---- */
+
+#define N 65536
+static float g_series[N];
+static struct event g_ev[8];
+
+static accel_search *handle(void)
+{
+    accel_search *s = (accel_search *) calloc(1, sizeof(*s));
+    s->g.numbins = N / 2;
+    s->g.dt = 1e-3;
+    s->stream = (void *) 1;
+    s->stream2 = (void *) 2;
+    s->ev_norms = &g_ev[0];
+    CHECK(agpu_malloc(&s->d_spec, sizeof(accel_fcomplex) * N / 2) == 0);
+    s->own_spec = 1;
+    g_nop = 0;
+    g_fail = "";
+    return s;
+}
+
+static void drop(accel_search *s)
+{
+    done(s->stream, g_nop);
+    done(s->stream2, g_nop);
+    if (s->own_spec)
+        agpu_free(s->d_spec);
+    agpu_free(s->d_fftwork);
+    agpu_free(s->d_dblk);
+    agpu_free(s->d_dmean);
+    free(s);
+}
+
+/* The handle's own spectrum is freed only when nothing reads or writes it:
+ * neither a preparation on the handle's stream nor norms on the second. */
+static void spectrum_replaced(void)
+{
+    accel_fcomplex other;
+    for (int k = 0; k < 3; k++) {
+        accel_search *s = handle();
+        if (k == 0)
+            CHECK(accel_search_set_series(s, g_series, N) == 0);
+        if (k == 1)
+            CHECK(accel_search_set_device_series(s, g_series, N) == 0);
+        if (k == 2)
+            op(s->stream2, s->d_spec, NULL);
+        CHECK(accel_search_set_device_spectrum(s, &other) == 0);
+        CHECK(s->d_spec == &other && !s->own_spec);
+        drop(s);
+    }
+}
+
+int main(void)
+{
+    spectrum_replaced();
+    printf("series checks passed\n");
+    return 0;
+}

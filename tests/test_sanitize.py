@@ -63,3 +63,22 @@ def test_request_loop_under_sanitizer(tmp_path, sanitizer):
     assert r.returncode == 0, (r.stdout + r.stderr)[-4000:]
     assert "request loop checks passed" in r.stdout
     assert "ThreadSanitizer" not in r.stderr and "runtime error" not in r.stderr
+
+
+@pytest.mark.skipif(shutil.which("gcc") is None, reason="gcc not available")
+def test_series_setters_and_streams(tmp_path):
+    """The setters of a search handle's series and spectrum with test doubles
+    of the device layer that book which operation is pending on which buffer
+    (tests/sanitize/series_driver.c)."""
+    exe = tmp_path / "series_driver"
+    cmd = ["gcc", "-O1", "-g", "-std=gnu11", "-fsanitize=address,undefined",
+           "-fno-sanitize-recover=all", "-fno-omit-frame-pointer", "-ffunction-sections",
+           "-fdata-sections", "-I", CSRC, "-I", os.path.join(ROOT, "include"),
+           os.path.join(ROOT, "tests", "sanitize", "series_driver.c")] + \
+          [os.path.join(CSRC, f) for f in HOST_SOURCES if f != "accel_host.c"] + \
+          ["-Wl,--gc-sections", "-lm", "-lpthread", "-o", str(exe)]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr[-3000:]
+    r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0, (r.stdout + r.stderr)[-4000:]
+    assert "series checks passed" in r.stdout
