@@ -2002,16 +2002,18 @@ static int set_series(accel_search *s, const float *series, long long n, int on_
     }
     /* realfft (src/accel_utils.c:1547), deredden (:1561), bin 0 := 1+1i
      * (:1621-1624; left as de-reddened under -photon), all on the device */
-    if (on_device) {
-        /* the caller's series is free once the copy is done; the rest runs on */
-        GPU(agpu_copy_d2d(s->d_spec, series, sizeof(float) * (size_t) n, s->stream));
-        GPU(agpu_event_record(s->ev_norms, s->stream));
-    } else {
-        GPU(agpu_h2d(s->d_spec, series, sizeof(float) * (size_t) n, s->stream));
+    int rc = on_device ? agpu_copy_d2d(s->d_spec, series, sizeof(float) * (size_t) n, s->stream) ||
+                             agpu_event_record(s->ev_norms, s->stream)
+                       : agpu_h2d(s->d_spec, series, sizeof(float) * (size_t) n, s->stream);
+    rc = rc || agpu_realfft((const float *) s->d_spec, n, s->d_spec, s->d_fftwork, s->stream) ||
+         agpu_deredden(s->d_spec, g->numbins, s->d_dblk, s->ndblk, s->dmaxn, s->d_dmean,
+                       s->p.nph > 0.0 ? 0.0f : 1.0f, s->stream);
+    if (rc) {
+        set_err("accel_search_set_series: %s", agpu_last_error());
+        agpu_stream_sync(s->stream);   /* the copy of the caller's series may still run */
+        return -1;
     }
-    GPU(agpu_realfft((const float *) s->d_spec, n, s->d_spec, s->d_fftwork, s->stream));
-    GPU(agpu_deredden(s->d_spec, g->numbins, s->d_dblk, s->ndblk, s->dmaxn, s->d_dmean,
-                      s->p.nph > 0.0 ? 0.0f : 1.0f, s->stream));
+    /* the caller's series is free once the copy is done; the rest runs on */
     if (on_device)
         GPU(agpu_event_sync(s->ev_norms));
     return 0;

@@ -156,9 +156,26 @@ static void spectrum_replaced(void)
     }
 }
 
+/* The caller may free a device series when the call returns, also when the
+ * preparation fails. */
+static void series_returned(void)
+{
+    accel_search *s = handle();
+    CHECK(accel_search_set_device_series(s, g_series, N) == 0);
+    CHECK(!pending(g_series));
+    drop(s);
+    s = handle();
+    g_fail = "realfft";
+    CHECK(accel_search_set_device_series(s, g_series, N) != 0);
+    CHECK(strstr(accel_last_error(), "double"));
+    CHECK(!pending(g_series));
+    drop(s);
+}
+
 int main(void)
 {
     spectrum_replaced();
+    series_returned();
     printf("series checks passed\n");
     return 0;
 }
