@@ -316,6 +316,8 @@ struct accel_search {
     void *stream2;                    /* the block norms, beside the correlation */
     void *ev[5];
     void *ev_norms;
+    void *ev_copy;                    /* a device series' copy (not a search's event: a
+                                       * launched search may be uncollected) */
     void *d_spec;
     int own_spec;
     void *d_T;
@@ -686,6 +688,7 @@ static int search_init(accel_search *s, int device, int nstreams)
     for (int i = 0; i < 5; i++)
         GPU(agpu_event_create(&s->ev[i]));
     GPU(agpu_event_create(&s->ev_norms));
+    GPU(agpu_event_create(&s->ev_copy));
     s->numw1 = g->numw ? g->numw : 1;
     s->nt = s->numw1 * g->numz;
     s->hw = g->maxkernlen / (2 * ACCEL_NUMBETWEEN);
@@ -827,6 +830,8 @@ void accel_search_destroy(accel_search *s)
             agpu_event_destroy(s->ev[i]);
     if (s->ev_norms)
         agpu_event_destroy(s->ev_norms);
+    if (s->ev_copy)
+        agpu_event_destroy(s->ev_copy);
     if (s->stream)
         agpu_stream_destroy(s->stream);
     if (s->stream2 && s->stream2 != s->stream)
@@ -2003,7 +2008,7 @@ static int set_series(accel_search *s, const float *series, long long n, int on_
     /* realfft (src/accel_utils.c:1547), deredden (:1561), bin 0 := 1+1i
      * (:1621-1624; left as de-reddened under -photon), all on the device */
     int rc = on_device ? agpu_copy_d2d(s->d_spec, series, sizeof(float) * (size_t) n, s->stream) ||
-                             agpu_event_record(s->ev_norms, s->stream)
+                             agpu_event_record(s->ev_copy, s->stream)
                        : agpu_h2d(s->d_spec, series, sizeof(float) * (size_t) n, s->stream);
     rc = rc || agpu_realfft((const float *) s->d_spec, n, s->d_spec, s->d_fftwork, s->stream) ||
          agpu_deredden(s->d_spec, g->numbins, s->d_dblk, s->ndblk, s->dmaxn, s->d_dmean,
@@ -2015,7 +2020,7 @@ static int set_series(accel_search *s, const float *series, long long n, int on_
     }
     /* the caller's series is free once the copy is done; the rest runs on */
     if (on_device)
-        GPU(agpu_event_sync(s->ev_norms));
+        GPU(agpu_event_sync(s->ev_copy));
     return 0;
 }
 

@@ -118,6 +118,7 @@ static accel_search *handle(void)
     s->stream = (void *) 1;
     s->stream2 = (void *) 2;
     s->ev_norms = &g_ev[0];
+    s->ev_copy = &g_ev[1];
     CHECK(agpu_malloc(&s->d_spec, sizeof(accel_fcomplex) * N / 2) == 0);
     s->own_spec = 1;
     g_nop = 0;
@@ -172,8 +173,20 @@ static void series_returned(void)
     drop(s);
 }
 
+/* The next series may be set while a search is launched and not collected:
+ * the events that its timings come from stay as they are. */
+static void launched_search(void)
+{
+    accel_search *s = handle();
+    agpu_event_record(s->ev_norms, s->stream2);
+    CHECK(accel_search_set_device_series(s, g_series, N) == 0);
+    CHECK(g_ev[0].stream == s->stream2 && g_ev[0].mark == 0);
+    drop(s);
+}
+
 int main(void)
 {
+    launched_search();
     spectrum_replaced();
     series_returned();
     printf("series checks passed\n");
