@@ -109,12 +109,16 @@ const accel_geom *accel_search_geom(const accel_search *s);
 /* Copies the spectrum (numbins complex values, first one at bin lobin) to
  * HBM.  Replaces the mmap / .dat read of create_accelobs. */
 int accel_search_set_spectrum(accel_search *s, const accel_fcomplex *fft);
-/* Takes a time series of n samples (n even, n/2 = numbins, lobin 0) and prepares its spectrum on the GPU as accelsearch prepares a
- * .dat: realfft, deredden and bin 0 := 1+1i (src/accel_utils.c:1507-1562,
- * 1621-1624). */
+/* Takes a time series of n samples (n even, n/2 = numbins, lobin 0) and
+ * prepares its spectrum on the GPU as accelsearch prepares a .dat: realfft,
+ * deredden and bin 0 := 1+1i (src/accel_utils.c:1507-1562, 1621-1624).  The
+ * spectrum is prepared when the call returns. */
 int accel_search_set_series(accel_search *s, const float *series, long long n);
 /* The same for a series already in device memory on the handle's device
- * (a DM trial of accel_dedisperse_dev): no host round trip. */
+ * (a DM trial of accel_dedisperse_dev): no host round trip.  When the call
+ * returns the series has been copied and may be freed or overwritten; the
+ * preparation goes on on the handle's stream, ahead of every later use of
+ * the spectrum through the handle. */
 int accel_search_set_device_series(accel_search *s, const float *d_series, long long n);
 /* Copies the first n bins of the search's current spectrum to the host. */
 int accel_search_spectrum(const accel_search *s, accel_fcomplex *out, long long n);

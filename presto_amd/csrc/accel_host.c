@@ -2018,9 +2018,12 @@ static int set_series(accel_search *s, const float *series, long long n, int on_
         agpu_stream_sync(s->stream);   /* the copy of the caller's series may still run */
         return -1;
     }
-    /* the caller's series is free once the copy is done; the rest runs on */
+    /* a device series is the caller's again once its copy is done, and the
+     * rest runs on; a host series' preparation ends here */
     if (on_device)
         GPU(agpu_event_sync(s->ev_copy));
+    else
+        GPU(agpu_stream_sync(s->stream));
     return 0;
 }
 

@@ -165,6 +165,12 @@ static void series_returned(void)
     CHECK(accel_search_set_device_series(s, g_series, N) == 0);
     CHECK(!pending(g_series));
     drop(s);
+    /* a host series is prepared when the call returns (a request's
+     * preparation time is measured around it) */
+    s = handle();
+    CHECK(accel_search_set_series(s, g_series, N) == 0);
+    CHECK(!pending(s->d_spec));
+    drop(s);
     s = handle();
     g_fail = "realfft";
     CHECK(accel_search_set_device_series(s, g_series, N) != 0);
