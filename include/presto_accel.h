@@ -161,10 +161,9 @@ int accel_search_plane_row(const accel_search *s, int wi, int zi, long long hb0,
 int accel_search_nwindows(const accel_search *s);
 int accel_search_norms(const accel_search *s, double *out, int n);
 /* Milliseconds of the last run (HIP events): block norms (on a second
- * stream, beside the correlation), correlation, the gap between the
- * correlation and the harmonic sum (the plane's halos or bounds are written by
- * the correlation, so about 0), harmonic sum (including any wait for the
- * norms), total. */
+ * stream, beside the correlation), correlation, 0 (the plane's halos or
+ * bounds, which the correlation writes), harmonic sum (including any wait for
+ * the norms), total (with the hits' sigmas, which follow the harmonic sum). */
 int accel_search_timings(const accel_search *s, float *ms5);
 /* Host wall-clock milliseconds of the last run: enqueueing the kernels,
  * waiting for them, copying the hits back, replaying the hits into the

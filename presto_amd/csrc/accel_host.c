@@ -926,13 +926,12 @@ int accel_search_launch(accel_search *s)
                        s->hb_end, s->d_plane, s->ntiles, s->groups, 0, -1, s->bounds,
                        s->stream));
     GPU(agpu_event_record(s->ev[2], s->stream));
-    /* the tile halos or bounds are written by the correlation itself */
-    GPU(agpu_event_record(s->ev[3], s->stream));
     if (two)
         GPU(agpu_stream_wait_event(s->stream, s->ev_norms));
     GPU(harmsum(s, &a));
-    GPU(agpu_event_record(s->ev[4], s->stream));
+    GPU(agpu_event_record(s->ev[3], s->stream));
     GPU(hit_sigmas(s));
+    GPU(agpu_event_record(s->ev[4], s->stream));
     s->hms[0] = now_ms() - t0;
     return 0;
 }
@@ -1164,8 +1163,9 @@ int accel_search_collect(accel_search *s)
         }
     }
     rc = rc || agpu_event_elapsed(&s->ms[0], s->ev[0], s->ev_norms);
-    for (int i = 1; i < 4; i++)
-        rc = rc || agpu_event_elapsed(&s->ms[i], s->ev[i], s->ev[i + 1]);
+    s->ms[2] = 0.0f;   /* the tile halos or bounds are written by the correlation itself */
+    rc = rc || agpu_event_elapsed(&s->ms[1], s->ev[1], s->ev[2]) ||
+         agpu_event_elapsed(&s->ms[3], s->ev[2], s->ev[3]);
     rc = rc || agpu_event_elapsed(&s->ms[4], s->ev[0], s->ev[4]);
     double t1 = now_ms();
     s->hms[1] = t1 - t0;

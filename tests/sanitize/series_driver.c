@@ -1,7 +1,7 @@
 /*
- * Host-only driver for what the series and spectrum setters of a search
- * handle (accel_host.c, included here so that a handle can be laid out by
- * hand) promise about memory and streams, built by tests/test_sanitize.py.
+ * Host-only driver for what a search handle (accel_host.c, included here so
+ * that a handle can be laid out by hand) promises about memory, streams and
+ * events, built by tests/test_sanitize.py.
  * The device layer is replaced by test doubles that only book: an operation
  * stays pending on its stream, with the buffers it reads and writes, until
  * the stream, or an event recorded behind it, is waited for.
@@ -104,6 +104,70 @@ int agpu_deredden(void *spec, long long numbins, const agpu_window *blk, int nbl
     return 0;
 }
 
+int agpu_memset(void *p, int v, size_t bytes, void *stream)
+{
+    (void) v, (void) bytes;
+    op(stream, NULL, p);
+    return 0;
+}
+int agpu_d2h(void *dst, const void *src, size_t bytes, void *stream)
+{
+    (void) src;
+    memset(dst, 0, bytes);   /* no hits */
+    return done(stream, g_nop);
+}
+int agpu_stream_wait_event(void *s, void *e) { return (void) s, (void) e, 0; }
+int agpu_event_elapsed(float *ms, void *start, void *stop)
+{
+    *ms = (float) (((struct event *) stop)->mark - ((struct event *) start)->mark);
+    return 0;
+}
+int agpu_block_norms(const void *spec, long long numbins, long long lobin, const agpu_window *win,
+                     int nwin, int maxn, double *norm, float *nsq, void *stream)
+{
+    (void) numbins, (void) lobin, (void) win, (void) nwin, (void) maxn, (void) norm, (void) nsq;
+    op(stream, spec, NULL);
+    return 0;
+}
+int agpu_correlate(const void *spec, long long numbins, long long lobin, const void *T, int nt,
+                   int L, int hw, int uselen, long long hb_end, float *plane, long long ntiles,
+                   int groups, long long seg_lo, long long seg_hi, int bounds, void *stream)
+{
+    (void) numbins, (void) lobin, (void) T, (void) nt, (void) L, (void) hw, (void) uselen;
+    (void) hb_end, (void) plane, (void) ntiles, (void) groups, (void) seg_lo, (void) seg_hi;
+    (void) bounds;
+    op(stream, spec, NULL);
+    return 0;
+}
+int agpu_harmsum(const agpu_harmsum_args *a, long long c_lo, long long c_hi, void *stream)
+{
+    (void) a, (void) c_lo, (void) c_hi;
+    op(stream, NULL, NULL);
+    return 0;
+}
+int agpu_hit_sigmas(agpu_hitrec *hits, const unsigned *nhits, unsigned cap,
+                    const agpu_numindep *ni, void *stream)
+{
+    (void) nhits, (void) cap, (void) ni;
+    op(stream, NULL, hits);
+    return 0;
+}
+/* linked, not reached: no bounds, standard norms */
+int agpu_harmbound(const agpu_harmsum_args *a, const float *nb, void *stream)
+{
+    return (void) a, (void) nb, (void) stream, -1;
+}
+int agpu_bound_norms(const agpu_harmsum_args *a, long long hb_end, float *nb, void *stream)
+{
+    return (void) a, (void) hb_end, (void) nb, (void) stream, -1;
+}
+int agpu_inmem_nsq_table(const float *nsq, int npre, int nblocks, long long rh0, int cu,
+                         long long hb_end, float *out, void *stream)
+{
+    (void) nsq, (void) npre, (void) nblocks, (void) rh0, (void) cu, (void) hb_end, (void) out;
+    return (void) stream, -1;
+}
+
 /* ---- a handle with what the setters use ---- */
 
 #define N 65536
@@ -119,6 +183,8 @@ static accel_search *handle(void)
     s->stream2 = (void *) 2;
     s->ev_norms = &g_ev[0];
     s->ev_copy = &g_ev[1];
+    for (int i = 0; i < 5; i++)
+        s->ev[i] = &g_ev[2 + i];
     CHECK(agpu_malloc(&s->d_spec, sizeof(accel_fcomplex) * N / 2) == 0);
     s->own_spec = 1;
     g_nop = 0;
@@ -190,8 +256,28 @@ static void launched_search(void)
     drop(s);
 }
 
+/* The times of a search: one unit per operation between two events. */
+static void timings(void)
+{
+    accel_search *s = handle();
+    agpu_hitrec hits[2];
+    float ms[5];
+    s->d_hits = hits + 1;
+    s->d_nhits = (unsigned *) hits;
+    s->cap = 1;
+    s->g.numharmstages = 1;
+    CHECK(accel_search_launch(s) == 0 && accel_search_collect(s) == 0);
+    CHECK(accel_search_timings(s, ms) == 0);
+    CHECK(ms[0] == 1 && ms[1] == 1 && ms[2] == 0 && ms[3] == 1);
+    CHECK(ms[4] == 4);   /* norms, correlation, harmonic sum and sigmas */
+    free(s->hits);
+    free(s->sigs);
+    drop(s);
+}
+
 int main(void)
 {
+    timings();
     launched_search();
     spectrum_replaced();
     series_returned();

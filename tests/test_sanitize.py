@@ -67,9 +67,9 @@ def test_request_loop_under_sanitizer(tmp_path, sanitizer):
 
 @pytest.mark.skipif(shutil.which("gcc") is None, reason="gcc not available")
 def test_series_setters_and_streams(tmp_path):
-    """The setters of a search handle's series and spectrum with test doubles
-    of the device layer that book which operation is pending on which buffer
-    (tests/sanitize/series_driver.c)."""
+    """The setters of a search handle's series and spectrum and the events of
+    its times with test doubles of the device layer that book which operation
+    is pending on which buffer (tests/sanitize/series_driver.c)."""
     exe = tmp_path / "series_driver"
     cmd = ["gcc", "-O1", "-g", "-std=gnu11", "-fsanitize=address,undefined",
            "-fno-sanitize-recover=all", "-fno-omit-frame-pointer", "-ffunction-sections",
