@@ -383,6 +383,9 @@ typedef struct {
 int agpu_fold_search(const agpu_fold_search_args *args, void *stream);
 /* periods per tile of the search */
 int agpu_fold_tile(int npart, int proflen);
+/* workgroups of that search that the current device holds at once, -1 on
+ * failure */
+int agpu_fold_resident(int npart, int proflen);
 /* *d_first := the smallest index of the largest redchi above 0 of rows x
  * numtrials trials, 0 if there is none */
 int agpu_fold_first(const double *d_redchi, const unsigned long long *d_tilemax,

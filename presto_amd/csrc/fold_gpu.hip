@@ -232,10 +232,12 @@ __device__ static unsigned long long fs_redchi(const agpu_fold_search_args &a, c
  * workgroups as are resident: each reads the folds into LDS once, and a
  * tile's serial sums over the bins run in FS_TR lanes at once.  One workgroup
  * per trial (k_fold_search) re-read the folds and summed in a single lane:
- * 136 us for 257 x 257 trials of 64 parts by 64 bins, here 99.  Bound by the
+ * 136 us for 257 x 257 trials of 64 parts by 64 bins, here 83.  Bound by the
  * LDS reads of a sum (8 B per trial, part and bin: 30 us at 128 B a clock,
  * half as much again for the offsets) and by the latency of its chain, which
- * 16 waves per workgroup cover better than 4 (117 us). */
+ * 16 waves per workgroup cover better than 4, and two workgroups a CU better
+ * than one (97 us): the second launch bound holds the scalar registers to 8
+ * waves per SIMD (106 of them allow 7, so one workgroup of 4 per SIMD). */
 #define FS_TR 32
 #define FS_TH 1024
 #define FS_UN 8 /* parts per step of a sum: their loads are in flight together */
@@ -250,7 +252,7 @@ static size_t fs_tile_lds(int npart, int proflen)
            sizeof(int) * (size_t) FS_TR * fs_rows(npart);
 }
 
-__global__ __launch_bounds__(FS_TH) void k_fold_search_tile(agpu_fold_search_args a)
+__global__ __launch_bounds__(FS_TH, 8) void k_fold_search_tile(agpu_fold_search_args a)
 {
     extern __shared__ double fs_lds[];
     const int L = a.proflen, nt = a.numtrials, nr = fs_rows(a.npart);
@@ -356,6 +358,20 @@ extern "C" int agpu_fold_tile(int npart, int proflen)
     return fs_tile_lds(npart, proflen) <= 64 * 1024 ? FS_TR : 1;
 }
 
+/* workgroups of the tile kernel that the current device holds at once: a
+ * further one would read the folds again for tiles that a resident one could
+ * take (32 parts by 64 bins, 1024 instead of 512 workgroups: 63 us against
+ * 54, of which the second workgroup of a CU gives 8) */
+extern "C" int agpu_fold_resident(int npart, int proflen)
+{
+    int dev = 0, ncu = 0, per_cu = 0;
+    FD_CHECK(hipGetDevice(&dev));
+    FD_CHECK(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
+    FD_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_fold_search_tile, FS_TH,
+                                                          fs_tile_lds(npart, proflen)));
+    return ncu * (per_cu > 0 ? per_cu : 1);
+}
+
 extern "C" int agpu_fold_search(const agpu_fold_search_args *args, void *stream)
 {
     if (args->npart < 1 || args->proflen < 2 || args->numtrials < 1 ||
@@ -367,8 +383,9 @@ extern "C" int agpu_fold_search(const agpu_fold_search_args *args, void *stream)
      * than 64 bins or so) the folds stay in L2 */
     if (agpu_fold_tile(args->npart, args->proflen) == FS_TR) {
         const long tiles = (long) ((args->numtrials + FS_TR - 1) / FS_TR) * args->numtrials;
-        const long resident =
-            256L * (long) (160 * 1024 / fs_tile_lds(args->npart, args->proflen));
+        const long resident = agpu_fold_resident(args->npart, args->proflen);
+        if (resident < 0)
+            return -1;
         hipLaunchKernelGGL(k_fold_search_tile, dim3((unsigned) (tiles < resident ? tiles : resident)),
                            dim3(FS_TH), fs_tile_lds(args->npart, args->proflen),
                            (hipStream_t) stream, *args);

@@ -5,7 +5,9 @@ long double in the oracle as in the reference; statistics within 1e-12);
 the p / p-dot search's plane bit-equal to the oracle's, with the same best
 trial; and the end-to-end path accelsearch -> .cand -> fold -> search on
 the sifting fixtures' pulsar."""
+import ctypes
 import os
+import re
 import subprocess
 import sys
 
@@ -234,3 +236,15 @@ def test_gpu_fold_search_tiles(npart, nb, npfact, flat):
     assert np.array_equal(pp.view(np.uint32), want.view(np.uint32))
     assert (best.ip, best.ipd) == (wb["ip"], wb["ipd"])
     assert not flat or (best.ip, best.ipd) == (0, 0) and not pp.any()
+
+
+@pytest.mark.parametrize("npart,nb", [(64, 64), (64, 73), (32, 64), (8, 16)])
+def test_fold_search_workgroups_are_resident(npart, nb):
+    """The tile search launches as many workgroups as the device holds: two
+    of 1024 threads a CU for every size that takes it, however little LDS a
+    tile needs."""
+    name = ctypes.create_string_buffer(256)
+    assert A.lib.agpu_init(0) == 0 and A.lib.agpu_device_name(name, 256) == 0
+    cus = int(re.search(r"(\d+) CUs", name.value.decode()).group(1))
+    assert A.lib.agpu_fold_tile(npart, nb) == 32
+    assert A.lib.agpu_fold_resident(npart, nb) == 2 * cus
