@@ -52,11 +52,13 @@ int accel_batch_handles(const accel_batch *b)
     return b->n;
 }
 
-/* A handle for params p that is not holding the results of item `busy`. */
+/* A handle for params p that is not holding the results of item `busy`
+ * (-1: none is held). */
 static pooled *get_handle(accel_batch *b, const accel_params *p, int busy)
 {
     for (int i = 0; i < b->n; i++)
-        if (!memcmp(&b->pool[i].p, p, sizeof(*p)) && b->pool[i].last_item != busy)
+        if (!memcmp(&b->pool[i].p, p, sizeof(*p)) &&
+            (busy < 0 || b->pool[i].last_item != busy))
             return &b->pool[i];
     if (b->n == POOL_MAX)
         return NULL;

@@ -58,3 +58,16 @@ def test_batch_equals_separate_runs(tmp_path):
         else:
             assert not os.path.exists(tmp_path / f"bat{k}_ACCEL_50")
     assert all(t > 0 for t in ms)
+
+
+def test_a_kept_batch_reuses_its_handles():
+    """Runs of one and of three spectra on one batch: two handles per
+    geometry, not another one with every run (64 fill the pool)."""
+    p, fft = _trials()[1]
+    with A.Batch() as b:
+        counts = []
+        for n in (1, 1, 3, 1, 3, 3):
+            cands, _ = b.run([(p, fft, None, None)] * n, optimize=False)
+            assert all(np.array_equal(c, cands[0]) for c in cands)
+            counts.append(b.handles())
+    assert counts == [1, 1, 2, 2, 2, 2]
