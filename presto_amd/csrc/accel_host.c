@@ -880,6 +880,8 @@ int accel_search_set_device_spectrum(accel_search *s, const void *d_fft)
     return 0;
 }
 
+int accel_search_uses_bounds(const accel_search *s) { return s->bounds; }
+
 static int harmsum(accel_search *s, const agpu_harmsum_args *a)
 {
     return s->bounds ? agpu_harmbound(a, s->d_nb, s->stream) : agpu_harmsum(a, 0, -1, s->stream);

@@ -32,6 +32,9 @@ ACCEL_HIDDEN void accel_search_dev_view(const accel_search *s, accel_dev_view *v
  * streams per handle would share the device's few hardware queues). */
 ACCEL_HIDDEN accel_search *accel_search_create_streams(const accel_params *p, int device,
                                                        int nstreams);
+/* 1 if the search sums by bounds (agpu_harmbound), 0 if every cell
+ * (agpu_harmsum).  Not hidden: the tests ask it. */
+int accel_search_uses_bounds(const accel_search *s);
 /* The raw plane alone (correlation and halos over every half-bin), then
  * waits for it. */
 ACCEL_HIDDEN int accel_search_plane_only(accel_search *s);

@@ -2,9 +2,9 @@
 every hit recomputed in numpy from the search's raw plane and norms, term by
 term in FP32 in the order of the fractions, so set and powers must be equal.
 The shapes are those at which it can go wrong: 1 to 5 stages, both index
-rules, row blocks below, at and above 64 rows, jerk rows, ragged lengths, a
-first half-bin off every chunk edge, strong signals, bins without power,
-infinities and NaN."""
+rules, one, two and four blocks of z rows, jerk rows, ragged lengths, a first
+half-bin off every chunk edge, a last one inside a run, strong signals, bins
+without power, infinities and NaN.  The handle says which kernel it runs."""
 import ctypes as C
 
 import numpy as np
@@ -13,13 +13,11 @@ import pytest
 pytestmark = pytest.mark.gpu
 A = pytest.importorskip("presto_amd.accel")
 
-# agpu_harmbound_pays: thresholds high enough for their harmonics, 16 rows, 2^23 cells
-def _by_bounds(g):
-    numw = max(g.numw, 1)
-    cells = g.numz * numw * g.nblocks * g.corr_uselen
-    H = 2.0 ** np.arange(g.numharmstages)
-    cut = np.array(list(g.powcut))[:g.numharmstages]
-    return g.numz >= 16 and cells >= 1 << 23 and bool((cut >= 2.13 * H + 3.1 * np.sqrt(H)).all())
+
+def _by_bounds(s):
+    """Whether k_harmbound runs, as the handle itself says."""
+    A.lib.accel_search_uses_bounds.argtypes = [C.c_void_p]
+    return A.lib.accel_search_uses_bounds(s.h) == 1
 
 
 def _nearest(x):
@@ -93,6 +91,8 @@ def _spectrum(nbins, seed, signals=(), odd=None):
     (1 << 18, 100, None, 16, False, 77, None),
     (1 << 18, 100, None, 16, True, 1, None),
     (60000, 30, 40, 8, False, 50, None),              # 31 x 5 rows
+    (45001, 200, None, 8, True, 50, None),            # 201 rows, four blocks of 51 or 48
+    (45001, 200, None, 16, False, 50, None),
 ])
 def test_hits_equal_the_sums(nbins, zmax, wmax, numharm, inmem, rlo, odd):
     sig = [(nbins // 7, 9.0), (2 * (nbins // 7), 8.0), (3 * (nbins // 7), 7.0),
@@ -101,7 +101,7 @@ def test_hits_equal_the_sums(nbins, zmax, wmax, numharm, inmem, rlo, odd):
                       rlo=rlo, rhi=nbins - 1, inmem=inmem, force_standard=not inmem,
                       dat_input=False)
     with A.Search(p) as s:
-        assert _by_bounds(s.geom) and bool(s.geom.inmem) == inmem
+        assert _by_bounds(s) and bool(s.geom.inmem) == inmem
         s.set_spectrum(_spectrum(nbins, 11 + numharm, sig, odd))
         s.run()
         got = [(int(h["block"]), int(h["stage"]), int(h["wi"]), int(h["zi"]), int(h["ii"]),
@@ -143,7 +143,7 @@ def test_the_last_half_bins_in_used_memory(used_memory, numharm, inmem):
     run = end // 64 * 64
     assert 16 <= end - run <= 48
     with A.Search(p) as s:
-        assert _by_bounds(s.geom)
+        assert _by_bounds(s)
         s.set_spectrum(_spectrum(nbins, 5, [(run // 2 + 2, 40.0)]))
         s.run()
         got = [(int(h["block"]), int(h["stage"]), int(h["wi"]), int(h["zi"]), int(h["ii"]),
@@ -163,7 +163,7 @@ def test_nan_beside_a_signal(bits):
     p = A.make_params(nbins, 2 * nbins, 1e-3, zmax=40, numharm=1, sigma=2.5, rlo=100,
                       rhi=nbins - 1, force_standard=True, dat_input=False)
     with A.Search(p) as s:
-        assert _by_bounds(s.geom)
+        assert _by_bounds(s)
         uselen = s.corr_shape()["uselen"]
         hw = (4096 - uselen) // 4
         end = next(e for e in range(20 * uselen, 60 * uselen, uselen) if 16 <= e % 64 <= 48)
@@ -181,3 +181,22 @@ def test_nan_beside_a_signal(bits):
     near = [h for h in want
             if end <= 200 + h[0] * s.geom.corr_uselen + h[4] < (end // 64 + 1) * 64]
     assert len(near) > 5 and got == want
+
+
+@pytest.mark.parametrize("kw", [
+    dict(numharm=32), dict(zmax=14, nbins=300000), dict(nbins=60000), dict(sigma=1.0, numharm=16),
+    dict(rlo=100.5), dict(rlo=100.25)])
+def test_searches_that_sum_every_cell(kw):
+    """32 harmonics, 15 rows (one less than the rule asks), few cells, a low
+    threshold and starts off whole bins do not take the bounds; the in-memory
+    rule takes no half-bin start's lookups, so that one does."""
+    nbins = kw.pop("nbins", 150000)
+    kw = dict(dict(zmax=30, numharm=8, sigma=2.5, rlo=100), **kw)
+    p = A.make_params(nbins, 2 * nbins, 1e-3, rhi=nbins - 1, force_standard=True,
+                      dat_input=False, **kw)
+    with A.Search(p) as s:
+        assert s.geom.numz == kw["zmax"] + 1 and not _by_bounds(s)
+    if kw["rlo"] == 100.5:
+        p.force_standard, p.inmem = 0, 1
+        with A.Search(p) as s:
+            assert s.geom.inmem and _by_bounds(s)
