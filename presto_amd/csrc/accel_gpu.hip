@@ -675,8 +675,6 @@ __device__ static float2 unit_root(int a, int n)
     return make_float2((float) c, (float) s);
 }
 
-/* LDS slot of point i: one slot of padding every 16.  LPR(i, r): of point
- * i + r, r a multiple of 16 (an immediate offset from i's slot) */
 /* Stores through a buffer descriptor: a 32-bit byte offset from a base that
  * all lanes share, and the offset OFF_NONE is out of range, so the hardware
  * drops that lane's store. */
@@ -696,6 +694,8 @@ __device__ __forceinline__ void store_bound(__amdgpu_buffer_rsrc_t r, unsigned o
     __builtin_amdgcn_raw_buffer_store_b16((unsigned short) v, r, (int) off, 0, 0);
 }
 
+/* LDS slot of point i: one slot of padding every 16.  LPR(i, r): of point
+ * i + r, r a multiple of 16 (an immediate offset from i's slot) */
 #define LP(i) ((i) + ((i) >> 4))
 #define LPR(i, r) (LP(i) + (r) + (r) / 16)
 #define FFT_HALF (CORR_N / 2)
@@ -1569,7 +1569,10 @@ __host__ __device__ __forceinline__ int hb_zmap(int z, int k, int s)
     return m < 0 ? -((h - m) >> s) : (h + m) >> s;
 }
 
-/* any of the 16 sums above the threshold, or NaN */
+/* any of the 16 sums above the threshold, or NaN.  By their bits, which order
+ * like the sums since none is negative: bounds are powers, +inf or 0x7fff
+ * (k_corr), or 0 past the last half-bin (k_clear_bounds), and norms are
+ * squares. */
 __device__ __forceinline__ bool hb_over(const float *acc, float cut)
 {
     unsigned m = __float_as_uint(acc[0]);
@@ -2228,7 +2231,7 @@ int agpu_harmsum(const agpu_harmsum_args *a, long long c_lo, long long c_hi, voi
     if (a->nfrac + 1 > 32)
         return fail("agpu_harmsum: at most 31 sub-harmonic fractions");
     if (a->corr_uselen < HS_CHUNK / 2)
-        return fail("agpu_harmsum: corr_uselen below 1024 half-bins");
+        return fail("agpu_harmsum: corr_uselen below 512 half-bins");
     if (a->inmem && !a->nsq_hb)
         return fail("agpu_harmsum: in-memory path needs the per-half-bin norm table");
     if (a->rh_off < 0 || a->rh_off > 1 || (a->inmem && (a->rh_off || a->bstart)))

@@ -35,8 +35,8 @@ ACCEL_HIDDEN accel_search *accel_search_create_streams(const accel_params *p, in
 /* 1 if the search sums by bounds (agpu_harmbound), 0 if every cell
  * (agpu_harmsum).  Not hidden: the tests ask it. */
 int accel_search_uses_bounds(const accel_search *s);
-/* The raw plane alone (correlation and halos over every half-bin), then
- * waits for it. */
+/* The raw plane alone (correlation with halos or bounds over every
+ * half-bin), then waits for it. */
 ACCEL_HIDDEN int accel_search_plane_only(accel_search *s);
 /* Harmonic-polished refinement of n candidates on the handle's resident
  * spectrum (rin relative to lobin; win NULL for rz); pows and derivs are

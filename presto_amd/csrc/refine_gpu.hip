@@ -234,11 +234,14 @@ __device__ static void derivs_wg(const float2 *spec, long long numdata, double r
  * order, so all of them hold the same value and take the same simplex
  * step.  The local powers before and the powers and derivatives after
  * the simplex are per harmonic too, their interpolations dealt to the
- * workgroup's waves.  Latency-bound: an evaluation takes 4.5 us alone (one
- * tap per thread) and 6.5 us with 16 workgroups in step; 8 candidates of a
- * 2^21-sample, zmax 200 search take 0.98 ms (1.19 with a trip to memory per
- * harmonic's term, ten barriers per sum and the local powers' 20
- * interpolations one after another).  The launcher sizes each launch so
+ * workgroup's waves.  Latency-bound while a thread has one tap, that is
+ * 2 (0.55 (|z| H + 4) + 16) <= 256: |z| H, the z of the highest harmonic, up
+ * to 200, as in any candidate of a search with zmax <= 200.  There an
+ * evaluation takes 4.5 us alone and 6.5 us with 16 workgroups in step; 8
+ * candidates of a 2^21-sample, zmax 200 search take 0.98 ms (1.19 with a trip
+ * to memory per harmonic's term, ten barriers per sum and the local powers'
+ * 20 interpolations one after another).  Beyond, the FP64 work of a thread's
+ * taps in the first simplex grows in proportion to |z| H.  The launcher sizes each launch so
  * that all its workgroups can be resident at once; the barrier's wait is
  * bounded (RZ_SPIN_LIMIT polls), a group whose wait runs out is marked bad
  * and stops, and the launcher runs that candidate again on its own. */
