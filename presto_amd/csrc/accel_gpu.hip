@@ -900,23 +900,26 @@ __global__ __launch_bounds__(256, 4) void k_corr(const float2 *spec, long long n
         }
         if (BOUNDS) {
             /* the group's largest power rounded up to 16 bits: an upper bound
-             * that the harmonic sum looks at before it reads the powers.  Bit
-             * patterns, which order like the powers.  A NaN, whose bits reach
-             * up to ~0u, must not carry out of the rounding: any above
-             * 0x7fff0000 becomes the positive NaN 0x7fff */
+             * that the harmonic sum looks at before it reads the powers.  By
+             * their bits as signed numbers, which order like the powers.  A
+             * positive NaN is above all and must not carry into the sign, so
+             * the addition saturates; a negative one is below all, and a
+             * group of nothing else becomes a NaN or 0: no cell of it can
+             * cross, so either will do */
             int e = eg;
             asm volatile("" : "+v"(e));   /* see below */
 #pragma unroll
             for (int m = 0; m < 4; m++) {
-                unsigned w[2];
+                int w[2];
 #pragma unroll
                 for (int h = 0; h < 2; h++) {
-                    const unsigned x = max(__float_as_uint(p[2 * m + h].x),
-                                           __float_as_uint(p[2 * m + h].y));
-                    w[h] = max(x, (unsigned) __builtin_amdgcn_update_dpp(
-                                      0, (int) x, 0xb1 /* lanes 1,0,3,2 */, 0xf, 0xf, true));
+                    const int x = max(__float_as_int(p[2 * m + h].x),
+                                      __float_as_int(p[2 * m + h].y));
+                    w[h] = max(x, __builtin_amdgcn_update_dpp(
+                                      0, x, 0xb1 /* lanes 1,0,3,2 */, 0xf, 0xf, true));
                 }
-                const unsigned bnd = (min(tid & 1 ? w[1] : w[0], 0x7fff0000u) + 0xffffu) >> 16;
+                const unsigned bnd =
+                    (unsigned) __builtin_elementwise_add_sat(tid & 1 ? w[1] : w[0], 0xffff) >> 16;
                 store_bound(row, goff[m], bnd);
                 if (halo) {
                     const unsigned g = (unsigned) (e + 1024 * m) / AGPU_GROUP;
@@ -1570,9 +1573,9 @@ __host__ __device__ __forceinline__ int hb_zmap(int z, int k, int s)
 }
 
 /* any of the 16 sums above the threshold, or NaN.  By their bits, which order
- * like the sums since none is negative: bounds are powers, +inf or 0x7fff
- * (k_corr), or 0 past the last half-bin (k_clear_bounds), and norms are
- * squares. */
+ * like the sums since none is negative (a NaN of either sign exceeds every
+ * one): bounds are powers or NaN (k_corr), or 0 past the last half-bin
+ * (k_clear_bounds), and norms are squares. */
 __device__ __forceinline__ bool hb_over(const float *acc, float cut)
 {
     unsigned m = __float_as_uint(acc[0]);
