@@ -246,5 +246,5 @@ def test_fold_search_workgroups_are_resident(npart, nb):
     name = ctypes.create_string_buffer(256)
     assert A.lib.agpu_init(0) == 0 and A.lib.agpu_device_name(name, 256) == 0
     cus = int(re.search(r"(\d+) CUs", name.value.decode()).group(1))
-    assert A.lib.agpu_fold_tile(npart, nb) == 32
+    assert A.lib.agpu_fold_tile(npart, nb) == 32 and A.lib.agpu_fold_tile(64, 74) == 1
     assert A.lib.agpu_fold_resident(npart, nb) == 2 * cus
